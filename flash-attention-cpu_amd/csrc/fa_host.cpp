@@ -435,6 +435,20 @@ int make_plan(int variant, const void* q, const void* k, const void* v, const fl
         // splits beats several rounds of short ones.  The grid lists only
         // workgroups with keys.
         size_t per = 0;
+        // Folded grid (f32 v2 / v3, causal, at least two blocks per slice): a
+        // workgroup takes one half block from each end of the slice, so all
+        // of them have the same work.  Only where every block runs at once:
+        // a longer grid is evened out by starting its longest blocks first
+        // (map_block), and folding would make its last round a full one.
+        // Measured on MI355X (v3, causal): 16 x 2048^2 d128 247 -> 148 us,
+        // 32 x 1024^2 d128 126 -> 81, 16 x 2048^2 d64 130 -> 79.
+        const bool fold_ok = !lp && causal_skip && D <= kMaxDNarrow && nqb >= 2 && nqb * bh <= (size_t)num_cus;
+        // f32 v3 with 128-bit DMA and d = D = 128: pair query blocks nqb-1-r
+        // and r in one workgroup (equal causal work per workgroup; the
+        // second block's loads overlap the first's last step) when the
+        // pairs fill whole rounds of one workgroup per CU.
+        const bool pairs_ok = !lp && variant == 3 && vec && (size_t)D == d && D == 128 && nqb % 2 == 0 &&
+                              (nqb / 2 * bh) % (size_t)num_cus == 0;
         // The prefill splits' merge: the f32 split kernels at D = 64, 128,
         // 256 write their partial tiles in register order, merged a
         // workgroup per 16-row tile (a wave per 64 columns); the others
@@ -492,6 +506,15 @@ int make_plan(int variant, const void* q, const void* k, const void* v, const fl
             // workgroups resident at once: the 16-bit kernels fit two per CU at D <= 128
             const size_t resident = (size_t)num_cus * (lp && D <= 128 ? 2 : 1);
             bool stream = false;
+            // Most keys of a folded workgroup: half of its long and its short
+            // half block's (of `half` rows) together, largest for the pair in
+            // the middle of the slice (every pair's the same while sk >= sq).
+            auto fold_keys = [&](size_t half) -> double {
+                if (!causal_skip) return (double)sk;
+                const size_t nhb = (sq + half - 1) / half, r = (nhb - 1) / 2;
+                return 0.5 * (double)(std::min(sk, (nhb - r) * half) + std::min(sk, (r + 1) * half));
+            };
+            double best = 0.0;   // estimated time of the chosen plan, in keys of 128 rows
             if (path == FA_PATH_STREAM) {
                 if (opts->num_splits > 0 && (size_t)opts->num_splits > imax) return FA_ERR_UNSUPPORTED;
                 if (!stream_fit(opts->num_splits > 0 ? (size_t)opts->num_splits : resident)) return FA_ERR_UNSUPPORTED;
@@ -501,7 +524,10 @@ int make_plan(int variant, const void* q, const void* k, const void* v, const fl
                 per = (max_st + opts->num_splits - 1) / opts->num_splits;
             } else if (path == FA_PATH_AUTO && nqb * bh < (size_t)num_cus) {
                 const double cus = (double)num_cus, skd = (double)SKs;
-                double best = std::ceil((double)(nqb * bh) / cus) * (double)max_st * skd;   // no split
+                // no split: the longest block, or with the folded grid half
+                // the keys of its long and its short half block together
+                best = std::ceil((double)(nqb * bh) / cus) * (double)max_st * skd;
+                if (fold_ok) best = fold_keys(rows / 2);
                 // Candidates: for R = 1..4 rounds, the shortest split whose
                 // workgroups fit in R rounds (workgroup count falls as `per`
                 // grows, so bisect).
@@ -551,15 +577,11 @@ int make_plan(int variant, const void* q, const void* k, const void* v, const fl
             }
             if (per > 0 && (max_st + per - 1) / per < 2) per = 0;
             if (per > 0 && (bh * sq > imax || per * SKs > imax)) return FA_ERR_UNSUPPORTED;
-            // f32 v3 with 128-bit DMA and d = D = 128: pair query blocks nqb-1-r
-            // and r in one workgroup (equal causal work per workgroup; the
-            // second block's loads overlap the first's last step) when the
-            // pairs fill whole rounds of one workgroup per CU.
-            if (per == 0 && !lp && variant == 3 && vec && (size_t)D == d && D == 128 && nqb % 2 == 0 &&
-                (nqb / 2 * bh) % (size_t)num_cus == 0) {
+            if (per == 0 && pairs_ok) {
                 p.two_blocks = 1;
                 plan->first.gx = static_cast<unsigned>(nqb / 2 * bh);
             }
+            if (per == 0 && fold_ok && path == FA_PATH_AUTO && !p.two_blocks) p.fold = 1;
             if (per > 0) {
                 const size_t nks = (max_st + per - 1) / per;
                 if (nks > 65535 || nks > (size_t)kMaxSplits) return FA_ERR_UNSUPPORTED;

@@ -262,6 +262,9 @@ __device__ __forceinline__ void wait_vmcnt() {
     __builtin_amdgcn_s_waitcnt((N & 15) | ((N >> 4) << 14) | (7 << 4) | (15 << 8));
 }
 
+// Starts a new 64-byte line of code here (s_nop up to the boundary).
+__device__ __forceinline__ void align_code() { asm volatile(".p2align 6"); }
+
 // max / sum over the 4 lanes (l%16 + 16k) that hold one query row.  Both
 // swaps hand every lane the pair in the same order, so all 4 lanes end
 // with bit-identical results.
@@ -406,7 +409,18 @@ __device__ __forceinline__ void prefill_segment(const FaParams& p, const Prefill
     // + i], pre-multiplied by scale * log2(e) so scores come out of the MFMA
     // in the exp2 domain (src/v2.rs:171-173 multiplies after the dot; the
     // product differs by one f32 rounding per element of Q).
-    int row_first = q0 + 16 * tile;
+    // Folded grid (p.fold): the workgroup's lower tiles are half block
+    // nhb-1-qb (BQ / 2 rows), its upper tiles half block qb of the slice's nhb;
+    // with nhb odd the middle half block comes alone, and the upper tiles lie
+    // past seq_q.  Waves w and w + NW/2 share a SIMD, so every SIMD holds one
+    // long tile and one short one, and once the short tile is through, the
+    // long one has the SIMD to itself.
+    const bool fold = !STREAM && VARIANT != 1 && CG == 1 && p.fold != 0;
+    const int nhb = (seq_q + BQ / 2 - 1) / (BQ / 2);
+    const int row_a = !fold ? q0 + 16 * tile
+                      : tile < TILES / 2 ? (nhb - 1 - qb) * (BQ / 2) + 16 * tile
+                                         : (2 * qb + 1 == nhb ? nhb : qb) * (BQ / 2) + 16 * (tile - TILES / 2);
+    int row_first = row_a;
     int qrow = row_first + li;
     float qreg[NQ];
     auto load_q = [&](int row) {   // unscaled
@@ -452,7 +466,7 @@ __device__ __forceinline__ void prefill_segment(const FaParams& p, const Prefill
     // src/v1.rs:209-216); v2/v3 stop after the block's last diagonal key
     // (src/v2.rs:208-212, src/v3.rs:396-410).
     auto block_end = [&](int q0_) { return (VARIANT != 1 && causal) ? min(seq_k, q0_ + BQ) : seq_k; };
-    int kend = block_end(q0);
+    int kend = block_end(fold ? (nhb - 1 - qb) * (BQ / 2) - BQ / 2 : q0);
     // Key split / stream split (v2/v3 on grids smaller than the GPU): this
     // workgroup takes stages sbeg .. sbeg + nst - 1 of the block's range
     // (sbeg < the block's stage count by construction of the grid).
@@ -568,6 +582,14 @@ __device__ __forceinline__ void prefill_segment(const FaParams& p, const Prefill
     //    to that of the crate's 16-lane AVX-512 dot products
     //    (src/avx512.rs:195-234), which config 5's large logits need.
     constexpr bool BLOCKED_QK = D > 128;
+    // Each QK^T chunk and PV step of the v3 D = 128 kernel starts a 64-byte line
+    // of code.  Without it the loop's speed hangs on where the code before it
+    // happens to leave it: the same instructions 0 .. 31 words further on ran
+    // 32 x 2048^2 non-causal in 506 .. 518 us, causal in 269 .. 274; aligned,
+    // 505.6 and 268.2 wherever it starts.  Not on the other kernels (v2 d128
+    // 286.8 -> 293, v3 d64 141.8 -> 143, d256 unchanged: more s_nop between
+    // shorter chunks).
+    constexpr bool ALIGN = VARIANT == 3 && D == 128 && !STREAM;
     // Read-ahead: the first PRE d-chunks of the next QK^T and the first PRE
     // V steps of the next PV are read into registers before the softmax VALU
     // work (the stage is already resident), so their LDS latency is hidden;
@@ -632,6 +654,7 @@ __device__ __forceinline__ void prefill_segment(const FaParams& p, const Prefill
 #pragma unroll
             for (int cc = 0; cc < NC; ++cc) {
                 scale_chunk(cc);
+                if constexpr (ALIGN) align_code();
                 qk_mfma(kk[cc % KR], cc, s);
                 if (cc + PRE < NC) k_chunk(Ks, cc + PRE, kk[(cc + PRE) % KR]);
                 __builtin_amdgcn_sched_barrier(0);
@@ -645,6 +668,7 @@ __device__ __forceinline__ void prefill_segment(const FaParams& p, const Prefill
             for (int cc = 0; cc < NC; ++cc) {
                 if (cc + 1 < NC) k_chunk(Ks, cc + 1, kk[(cc + 1) & 1]);
                 scale_chunk(cc);
+                if constexpr (ALIGN) align_code();
                 qk_mfma(kk[cc & 1], cc, s);
                 __builtin_amdgcn_sched_barrier(0);
             }
@@ -796,6 +820,7 @@ __device__ __forceinline__ void prefill_segment(const FaParams& p, const Prefill
                 for (int hh = 0; hh < NVR; ++hh) vv[st][hh] = vpre[st][hh];
 #pragma unroll
             for (int step = 0; step < 4 * KB; ++step) {
+                if constexpr (ALIGN) align_code();
                 pv_step(step, vv[step % VR]);
                 if (step + PRE < 4 * KB) read_v(Vs, step + PRE, vv[(step + PRE) % VR]);
                 pv_hook(step);
@@ -806,6 +831,7 @@ __device__ __forceinline__ void prefill_segment(const FaParams& p, const Prefill
 #pragma unroll
             for (int step = 0; step < 4 * KB; ++step) {
                 read_v(Vs, step, vv);
+                if constexpr (ALIGN) align_code();
                 pv_step(step, vv);
                 pv_hook(step);
                 __builtin_amdgcn_sched_barrier(0);
@@ -924,7 +950,7 @@ __device__ __forceinline__ void prefill_segment(const FaParams& p, const Prefill
         auto kb_of = [&](int gs) { return gs < nA ? k0 + gs * SK : (gs - nA) * SK; };
         auto gstage_active = [&](int gs) -> bool {
             const int kbase = kb_of(gs);
-            const int rf = (gs < nA ? qb * BQ : q0_b) + 16 * tile;
+            const int rf = gs < nA ? row_a : q0_b + 16 * tile;
             return kbase < seq_k && !(causal && kbase > rf + 15);
         };
         if constexpr (LATE_Q) {

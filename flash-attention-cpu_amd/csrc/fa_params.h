@@ -32,6 +32,9 @@ typedef struct FaParams {
                          // block); 0 = plain longest-first order
     int two_blocks;      // f32 v3 prefill, d_head 128: each workgroup runs query blocks
                          // nqb-1-r and r of one (batch, head); nqb even, grid = bh * nqb / 2
+    int fold;            // f32 v2 / v3 prefill, causal: a workgroup's lower 64 rows are half block
+                         // nhb-1-r of the slice, its upper 64 rows half block r (equal work per
+                         // workgroup); 0 = 128 consecutive rows
     int full_keys;       // v1: every query block visits all seq_k keys, causal or not (no
                          // causal skip), so the key split, the stream split and fa_merge
                          // count each block's keys as the whole key range
