@@ -559,6 +559,53 @@ int make_plan(int variant, const void* q, const void* k, const void* v, const fl
                     }
                 }
             }
+            // Smaller workgroups (fa_fold.inc): 8 / G tiles of 16 rows, G
+            // waves sharing a tile's keys, no workspace and no merge launch.
+            // For grids that do not fill whole rounds of 128-row workgroups.
+            // Times in keys of 128 rows (0.128 us at D = 128, 0.0675 at 64),
+            // fitted to MI355X runs (v3): G = 4 9.0 us + 0.0351 us a key at
+            // D = 128, 6.8 + 0.0184 at 64; G = 2 9.2 + 0.0635, 7.9 + 0.0335
+            // (causal 256^2 .. 2048^2 and 1000 keys non-causal within 8 %).
+            // Before and after, us: 8 x 1000^2 d128 causal 46.1 -> 26.8
+            // (G = 4; key split before), 16 x 256^2 33.7 -> 12.6 (no split),
+            // 16 x 1024^2 59.8 -> 43.7 (G = 2; stream split), 8 x 2048^2 93.4
+            // -> 76.2, 8 x 1000^2 non-causal 49.7 -> 41.8, 20 x 2048^2 (320
+            // blocks of 128 rows) 252.6 -> 215.8.  At most 64 queries are the
+            // split-KV rule's above; up to 128 keys a block has two stages.
+            if (path == FA_PATH_AUTO && !lp && variant != 1 && vec && (D == 64 || D == 128) && !pairs_ok &&
+                sq > 64 && sk > 128 && nqb * bh <= 8 * (size_t)num_cus) {
+                const double cus = (double)num_cus;
+                if (nqb * bh >= (size_t)num_cus) {
+                    // one workgroup per block, longest first
+                    double total = 0.0;
+                    for (size_t b = 0; b < nqb; ++b) total += (double)block_stages(b);
+                    best = causal_skip ? std::max((double)max_st, total * (double)bh / cus) * (double)SKs
+                                       : std::ceil((double)(nqb * bh) / cus) * (double)sk;
+                    if (fold_ok) best = fold_keys(rows / 2);
+                }
+                // fixed costs that the estimates above leave out: a workgroup's
+                // start and end without a split (7 us at D = 128, 5 at 64),
+                // part of the second launch with one
+                best += stream || per > 0 ? (D == 64 ? 80.0 : 20.0) : (D == 64 ? 75.0 : 55.0);
+                int groups = 0;
+                for (int G = 2; G <= 4; G += 2) {
+                    const size_t half = (size_t)(64 / G), nhb = (sq + half - 1) / half, n = (nhb + 1) / 2 * bh;
+                    const double per_key = G == 2 ? 0.496 : 0.274, fixed = D == 64 ? (G == 2 ? 117.0 : 100.0) : 71.0;
+                    const double cost = std::ceil((double)n / cus) * (per_key * fold_keys(half) + fixed);
+                    if (n <= imax && cost < best) {
+                        best = cost;
+                        groups = G;
+                    }
+                }
+                if (groups) {
+                    std::snprintf(buf, sizeof(buf), "fa_prefill_v3_d%d_2k%d", D, groups);
+                    const size_t half = (size_t)(64 / groups), nhb = (sq + half - 1) / half;
+                    plan->first.name = buf;
+                    plan->first.gx = static_cast<unsigned>((nhb + 1) / 2 * bh);
+                    plan->first.bx = 512;
+                    return FA_OK;
+                }
+            }
             if (stream) {
                 plan->first.name += "s";   // the stream-split instantiation
                 plan->split = true;

@@ -2644,6 +2644,7 @@ FA_MERGE(2048)
 FA_NAIVE(float, f32)
 FA_NAIVE(double, f64)
 
+#include "fa_fold.inc"
 #include "fa_lp.inc"
 
 // ---------------------------------------------------------------------------

@@ -1,7 +1,8 @@
-"""Causal f32 prefills whose workgroups hold rows from both ends of a slice
-(the folded grid), at the sizes where the row mapping can go wrong: odd and
-even numbers of half blocks, ragged last half blocks, key ranges shorter and
-longer than the query range.  Against the oracle's CPU v2 under the parity
+"""f32 prefills whose workgroups hold rows from both ends of a slice (the folded
+grid), of 128 rows or of 2 or 4 16-row tiles whose keys several waves share,
+at the sizes where the row mapping can go wrong: odd and even numbers of half
+blocks, ragged last half blocks, key ranges shorter and longer than the query
+range, stages that only some of a tile's waves have keys of.  Against the oracle's CPU v2 under the parity
 bar of the other f32 tests (max-abs 2e-5, relative L2 1e-5)."""
 from __future__ import annotations
 
@@ -43,3 +44,61 @@ def test_folded_grid(shape, variant):
     plan = fa.describe_launch(variant, 1, bh, sq, sk, d, True)
     assert f"grid={-(-sq // 128) * bh}x1x1" in plan and "splits" not in plan, plan
     run(variant, bh, sq, sk, d, True)
+
+
+# 2 or 4 tiles of 16 rows per workgroup, 4 or 2 waves on each tile's keys
+# (stages of 64 keys at D = 128, 128 at D = 64)
+SMALL = [
+    # waves per tile, bh, sq, sk, d, causal
+    (4, 8, 129, 129, 64, True),      # 9 half blocks: the middle tile alone, one row in the last
+    (4, 8, 145, 145, 128, True),     # 10, one row in the last
+    (4, 3, 1000, 1000, 128, True),   # 63; stages of which only some waves have keys
+    (4, 8, 300, 700, 64, True),
+    (4, 8, 700, 200, 128, True),     # rows past the last key see them all
+    (4, 8, 300, 333, 100, False),    # d < D
+    (4, 8, 257, 129, 40, False),     # one key in the second stage, d < D
+    (2, 64, 200, 200, 128, True),    # 7 half blocks of 32 rows
+    (2, 64, 225, 225, 64, True),     # 8, one row in the last
+    (2, 64, 250, 140, 128, False),
+]
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("variant", (2, 3))
+@pytest.mark.parametrize("shape", SMALL)
+def test_shared_tiles(shape, variant):
+    groups, bh, sq, sk, d, causal = shape
+    plan = fa.describe_launch(variant, 1, bh, sq, sk, d, causal)
+    assert plan.startswith(f"fa_prefill_v3_d{64 if d <= 64 else 128}_2k{groups} "), plan
+    run(variant, bh, sq, sk, d, causal)
+
+
+@pytest.mark.gpu
+def test_shared_tiles_rows_without_mass():
+    """Scores of -inf (a key column of -inf against positive queries) weigh 0
+    in every wave's share, also where all of a wave's keys have them."""
+    bh, sq, d = 4, 200, 100
+    q, k, v = normal_vec(bh * sq * d, 1), normal_vec(bh * sq * d, 2), normal_vec(bh * sq * d, 3)
+    q.reshape(bh, sq, d)[:, :, 0] = 1.0
+    kk = k.reshape(bh, sq, d)
+    kk[:, 16:64, 0] = -np.inf   # whole shares of the first stage
+    kk[:, 150, 0] = -np.inf
+    out = np.full(bh * sq * d, np.nan, np.float32)
+    assert "_2k4 " in fa.describe_launch(3, 1, bh, sq, sq, d, False)
+    fa.flash_attention_multihead_v3(q, k, v, 1, bh, sq, sq, d, fa.FlashAttentionConfig(), out)
+    keep = np.isfinite(kk[0, :, 0])
+    want = np.concatenate([oracle.run(2, q.reshape(bh, -1)[h], np.ascontiguousarray(kk[h][keep]).ravel(),
+                                      np.ascontiguousarray(v.reshape(bh, sq, d)[h][keep]).ravel(), 1, sq,
+                                      int(keep.sum()), d, False, 64, 128) for h in range(bh)])
+    assert_parity(out, want, "keys of weight 0")
+
+
+def test_shared_tiles_are_planned_only_for_their_calls():
+    assert "_2k" not in fa.describe_launch(1, 1, 8, 1000, 1000, 128, True)            # v1: its own normalisation
+    assert "_2k" not in fa.describe_launch(3, 1, 8, 1000, 1000, 126, True)            # scalar loads
+    assert "_2k" not in fa.describe_launch(3, 1, 8, 1000, 1000, 256, True)
+    assert "_2k" not in fa.describe_launch(3, 1, 8, 1000, 1000, 128, True, fa.PATH_PREFILL)
+    assert "_2k" not in fa.describe_launch(3, 1, 8, 1000, 1000, 128, True, fa.PATH_STREAM)
+    assert "_2k" not in fa.describe_launch(3, 1, 8, 64, 1000, 128, False)             # split-KV's
+    assert "_2k" not in fa.describe_launch(3, 1, 32, 2048, 2048, 128, False)          # whole rounds
+    assert "_2k" not in fa.describe_launch(3, 1, 8, 1000, 1000, 128, True, dtype=fa.DTYPE_BF16)
