@@ -417,6 +417,44 @@ int make_plan(int variant, const void* q, const void* k, const void* v, const fl
             std::snprintf(buf, sizeof(buf), "fa_prefill_v%d_d%d_%d", variant, D, loader);
         }
         plan->first.name = buf;
+        // 16-bit query blocks of 2 .. 32 rows (16 at D = 256) against 256 keys or
+        // more: the streaming body of the split kernel, one workgroup per CU
+        // over all slices with at least kMinSplitKeys keys each; one split
+        // writes its rows directly.  (Causal, such a block sees 32 keys at
+        // most; below 256 keys the prefill body starts faster: 256 x 16 x 64
+        // 5.1 against 5.9 us.)  Measured on MI355X against the key-split
+        // prefill, bf16, us: 32 x 16 x 32768 d128 101.8 -> 83.2, 256 x 16 x
+        // 8192 186 -> 153 (7.0 TB/s), d64 114 -> 77, d256 32 x 16 x 32768 184
+        // -> 160; two workgroups per CU 83.8 / 161 / 84 / 187.  Two short
+        // splits lose to one: 128 x 16 x 1024 16.7 against 14.9.
+        const size_t few = D <= 128 ? 32 : 16;
+        if (lp && path == FA_PATH_AUTO && vec && D >= 64 && !causal && sq <= few && sk >= kMinSplitKeys) {
+            size_t n = std::max<size_t>(1, (size_t)num_cus / bh);
+            n = std::min(n, std::max<size_t>(1, sk / kMinSplitKeys));
+            if (n == 2 && sk < 2048) n = 1;
+            size_t len = ((sk + n - 1) / n + 63) / 64 * 64;
+            n = (sk + len - 1) / len;
+            if (n <= (size_t)kMaxSplits && len <= imax && bh * n <= imax && bh * sq <= imax) {
+                plan->first.name += "s";
+                plan->first.gx = static_cast<unsigned>(bh * n);
+                plan->first.bx = 64 * fa_lp_waves(lp_tiles);
+                p.few_rows = 1;
+                p.nqt = static_cast<int>(nqt);
+                p.num_splits = static_cast<int>(n);
+                p.split_len = static_cast<int>(len);
+                p.merge_scale = 1.0f;   // as the prefill's partials
+                plan->split = n > 1;
+                plan->ws_floats = 0;
+                if (n > 1) {
+                    std::snprintf(buf, sizeof(buf), "fa_merge_d%d", D);
+                    plan->second.name = buf;
+                    plan->second.gx = static_cast<unsigned>((bh * sq + FA_MERGE_ROWS - 1) / FA_MERGE_ROWS);
+                    plan->second.bx = 64 * FA_MERGE_ROWS;
+                    plan->ws_floats = bh * nqt * n * (16 * (size_t)D + 32);
+                }
+                return FA_OK;
+            }
+        }
         plan->first.gx = static_cast<unsigned>(nqb * bh);
         plan->first.bx = 64 * (lp ? fa_lp_waves(lp_tiles) : fa_prefill_waves(D));
         // The 16-bit kernels fit two workgroups per CU for D <= 128.
