@@ -560,6 +560,78 @@ int make_plan(int variant, const void* q, const void* k, const void* v, const fl
             } else if (opts && opts->num_splits > 1 && path == FA_PATH_PREFILL) {
                 if (opts->num_splits > kMaxSplits) return FA_ERR_UNSUPPORTED;
                 per = (max_st + opts->num_splits - 1) / opts->num_splits;
+            } else if (path == FA_PATH_AUTO && lp && vec && nqb * bh <= (size_t)num_cus) {
+                // 16-bit grids of at most one block per CU, estimated in us
+                // (MI355X, bf16; every shape of 1 .. 32 heads x 512 .. 4096
+                // within 15 %), fixed + per 64 keys: the plain kernel; 64, 96 or
+                // 128 rows with 4, 2, 2 waves on each tile's keys (D = 64, 128;
+                // causal: folded), where they all run at once; the key split,
+                // whose kernel is slower a stage (its segment loop) and which
+                // adds a merge launch and its partials, written and read back
+                // at 4 TB/s.  us before -> now: 16 x 1500^2 d64 36.9 -> 17.7 (96
+                // rows; key split before), 16 x 1024^2 23.8 -> 11.3 and d128 36.5
+                // -> 16.4 (64), causal 8 x 2048^2 33.4 -> 24.1 (64), 16 x 2048^2
+                // 41.2 -> 30.1 and 8 x 4096^2 75.4 -> 50.0 (128; plain before).
+                // The key split stays for few blocks of many keys: 1 x 2048^2
+                // d64 13.9 against 17.2.
+                const double cus = (double)num_cus, keys = (double)max_st;
+                const bool two = lp_tiles == 2;
+                const double fix = D == 32 ? 3.5 : D == 64 ? 3.6 : D == 128 ? 5.0 : 7.5;
+                const double plain = D == 32 ? 0.65 : D == 64 ? 0.80 : D == 128 ? (two ? 1.25 : 1.07) : 1.73;
+                const double split = D == 256 ? 1.9 : 1.19 * plain;
+                best = fix + plain * keys;
+                size_t wide = 0, wide_blocks = 0;   // rows and blocks (pairs of half blocks) per slice
+                bool wide_fold = false;
+                // (up to 128 keys a block has two stages)
+                if ((D == 64 || D == 128) && sk > 128) {
+                    const struct { size_t rows; double fixed, key64, causal64; } form[2][3] = {
+                        {{64, 4.8, 0.385, 0.37}, {96, 5.0, 0.50, 0.40}, {128, 5.0, 0.62, 0.43}},
+                        {{64, 6.6, 0.54, 0.51}, {96, 6.7, 0.72, 0.57}, {128, 6.5, 0.90, 0.62}}};
+                    for (const auto& f : form[D == 128]) {
+                        const size_t half = f.rows / 2, nhb = (sq + half - 1) / half;
+                        const bool fold = causal && nhb >= 2;
+                        const size_t nb = (nhb + 1) / 2;
+                        const double t = f.fixed + (fold ? f.causal64 : f.key64) * keys;
+                        if (nb * bh <= (size_t)num_cus && t < best) {
+                            best = t;
+                            wide = f.rows;
+                            wide_blocks = nb;
+                            wide_fold = fold;
+                        }
+                    }
+                }
+                for (size_t R = 1; R <= 4; ++R) {
+                    // the shortest split whose workgroups fit R per CU
+                    const size_t slots = R * (size_t)num_cus;
+                    size_t lo = 4, hi = max_st;
+                    if (lo > hi || wgs_for(hi) > slots) continue;
+                    while (lo < hi) {
+                        const size_t mid = (lo + hi) / 2;
+                        if (wgs_for(mid) <= slots) hi = mid;
+                        else lo = mid + 1;
+                    }
+                    if ((max_st + lo - 1) / lo < 2) continue;
+                    const double n = (double)wgs_for(lo);
+                    // two workgroups on a CU (D <= 128) take 1.5 times one's time
+                    const double turns = D <= 128 ? (n <= cus ? 1.0 : 1.5 * std::ceil(n / (2.0 * cus))) : std::ceil(n / cus);
+                    const double t = turns * (fix + split * (double)lo) + 5.5 + n * 128.0 * (4.0 * D + 8.0) * 2.0 / 4.0e6;
+                    if (t < best) {
+                        best = t;
+                        per = lo;
+                        wide = 0;
+                    }
+                }
+                if (wide) {
+                    std::snprintf(buf, sizeof(buf), "fa_prefill_lp_%s_d%d_2_t1r%d", dtype == FA_DTYPE_BF16 ? "bf16" : "f16", D,
+                                  static_cast<int>(wide));
+                    plan->first.name = buf;
+                    plan->first.gx = static_cast<unsigned>(wide_blocks * bh);
+                    plan->first.bx = wide == 96 ? 768 : 1024;
+                    p.nqb = static_cast<int>(wide_blocks);
+                    p.fold = wide_fold ? 1 : 0;
+                    p.pair_w = 0;
+                    return FA_OK;
+                }
             } else if (path == FA_PATH_AUTO && nqb * bh < (size_t)num_cus) {
                 const double cus = (double)num_cus, skd = (double)SKs;
                 // no split: the longest block, or with the folded grid half

@@ -1,0 +1,76 @@
+"""16-bit prefills of at most one 128-row block per CU: workgroups of 64, 96 or
+128 rows with 4, 2 and 2 waves on each 16-row tile's keys, causal ones folded
+(rows from both ends of the slice).  At the edges of half blocks, stages of 128
+keys and the waves' shares of them.  Against float64 attention on the same
+16-bit inputs under the 16-bit path's derived bound (probabilities rounded
+once: u / (1 - u) max|V|, u = 2^-8 bf16, 2^-11 f16, plus 2e-5 for the f32
+sums)."""
+from __future__ import annotations
+
+import numpy as np
+import pytest
+
+import flash_attention_amd as fa
+from fa_testutil import attention_f64, normal_vec, rel_l2
+
+DT = {"bf16": (fa.DTYPE_BF16, 2.0 ** -8), "f16": (fa.DTYPE_F16, 2.0 ** -11)}
+SHAPES = [
+    # rows, bh, sq, sk, d, causal
+    (64, 4, 300, 300, 64, True),      # 10 half blocks of 32 rows, 12 rows in the last
+    (64, 4, 289, 289, 128, True),     # 10, one row in the last: 5 pairs
+    (64, 4, 270, 270, 40, True),      # 9: the middle one alone, d < D
+    (64, 4, 700, 300, 64, True),      # keys end before the last queries
+    (64, 4, 300, 700, 104, True),     # keys past the last query, d < D
+    (64, 4, 129, 513, 128, False),    # one row in the third block, one key in the fifth stage
+    (64, 4, 100, 577, 64, False),     # the waves' shares of the last stage: 32, 32, 1 and no keys
+    (96, 64, 300, 300, 64, True),     # 7 half blocks of 48 rows: the middle one alone
+    (96, 64, 289, 289, 128, True),    # 7, one row in the last
+    (96, 64, 300, 193, 128, False),
+    (128, 64, 449, 449, 64, True),    # 8 half blocks of 64 rows, one row in the last
+    (128, 84, 300, 300, 128, True),   # 5: the middle one alone
+    (128, 64, 400, 321, 72, False),   # the second waves have one key of the last stage
+]
+
+
+def inputs(name, n, seed):
+    x = normal_vec(n, seed)
+    if name == "bf16":
+        bits = fa.f32_to_bf16_bits(x)
+        return bits, fa.bf16_bits_to_f32(bits)
+    h = x.astype(np.float16)
+    return h, h.astype(np.float32)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("name", sorted(DT))
+@pytest.mark.parametrize("shape", SHAPES)
+def test_shared_tiles(shape, name):
+    rows, bh, sq, sk, d, causal = shape
+    dt, u = DT[name]
+    plan = fa.describe_launch(2, 1, bh, sq, sk, d, causal, dtype=dt)
+    assert plan.startswith(f"fa_prefill_lp_{name}_d{64 if d <= 64 else 128}_2_t1r{rows} "), plan
+    q, qf = inputs(name, bh * sq * d, 1)
+    k, kf = inputs(name, bh * sk * d, 2)
+    v, vf = inputs(name, bh * sk * d, 3)
+    out = np.full(bh * sq * d, np.nan, np.float32)
+    fa.flash_attention_multihead_lp(dt, q, k, v, 1, bh, sq, sk, d, fa.FlashAttentionConfig(causal=causal), out)
+    want = np.concatenate([attention_f64(a, b, c, sq, sk, d, causal).ravel() for a, b, c in
+                           zip(qf.reshape(bh, -1), kf.reshape(bh, -1), vf.reshape(bh, -1))])
+    err = float(np.max(np.abs(out - want)))
+    assert np.all(np.isfinite(out))
+    assert err < u / (1 - u) * float(np.max(np.abs(vf))) + 2e-5, err
+    assert rel_l2(out, want) < u
+
+
+def test_shared_tiles_are_planned_only_for_their_calls():
+    def plan(*a, **kw):
+        return fa.describe_launch(2, 1, *a, dtype=fa.DTYPE_BF16, **kw)
+    assert "t1r96 grid=256x1x1 block=768" in plan(16, 1500, 1500, 64, False)
+    assert "t1r128 grid=256x1x1 block=1024" in plan(16, 2048, 2048, 128, True)
+    assert "t1r64 grid=256x1x1 block=1024" in plan(8, 2048, 2048, 64, True)
+    for other in (plan(17, 2048, 2048, 128, True), plan(32, 2048, 2048, 128, True),   # more blocks than CUs
+                  plan(8, 128, 128, 64, True), plan(8, 1000, 1000, 62, True),         # few keys, scalar loads
+                  plan(8, 1000, 1000, 256, True), plan(8, 1000, 1000, 32, True),
+                  plan(8, 1000, 1000, 64, True, path=fa.PATH_PREFILL), plan(8, 1000, 1000, 64, True, path=fa.PATH_STREAM),
+                  plan(1, 4096, 4096, 128, True)):                                    # few blocks of many keys: key split
+        assert "t1r" not in other, other
