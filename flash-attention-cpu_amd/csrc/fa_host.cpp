@@ -676,10 +676,10 @@ int make_plan(int variant, const void* q, const void* k, const void* v, const fl
             // fitted to MI355X runs (v3): G = 4 9.0 us + 0.0351 us a key at
             // D = 128, 6.8 + 0.0184 at 64; G = 2 9.2 + 0.0635, 7.9 + 0.0335
             // (causal 256^2 .. 2048^2 and 1000 keys non-causal within 8 %).
-            // Before and after, us: 8 x 1000^2 d128 causal 46.1 -> 26.8
-            // (G = 4; key split before), 16 x 256^2 33.7 -> 12.6 (no split),
-            // 16 x 1024^2 59.8 -> 43.7 (G = 2; stream split), 8 x 2048^2 93.4
-            // -> 76.2, 8 x 1000^2 non-causal 49.7 -> 41.8, 20 x 2048^2 (320
+            // Before and after, us: 8 x 1000^2 d128 causal 46.1 -> 26.2
+            // (G = 4; key split before), 16 x 256^2 33.7 -> 12.1 (no split),
+            // 16 x 1024^2 59.8 -> 43.0 (G = 2; stream split), 8 x 2048^2 93.4
+            // -> 76.0, 8 x 1000^2 non-causal 49.7 -> 41.0, 20 x 2048^2 (320
             // blocks of 128 rows) 252.6 -> 215.8.  At most 64 queries are the
             // split-KV rule's above; up to 128 keys a block has two stages.
             if (path == FA_PATH_AUTO && !lp && variant != 1 && vec && (D == 64 || D == 128) && !pairs_ok &&
