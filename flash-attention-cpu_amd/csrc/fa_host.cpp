@@ -418,10 +418,10 @@ int make_plan(int variant, const void* q, const void* k, const void* v, const fl
         }
         plan->first.name = buf;
         // 16-bit query blocks of 2 .. 32 rows (16 at D = 256) against 256 keys or
-        // more: the streaming body of the split kernel, one workgroup per CU
-        // over all slices with at least kMinSplitKeys keys each; one split
-        // writes its rows directly.  (Causal, such a block sees 32 keys at
-        // most; below 256 keys the prefill body starts faster: 256 x 16 x 64
+        // more: the streaming body (lp_rows_body), one workgroup per CU over
+        // all slices with at least kMinSplitKeys keys each; one split writes
+        // its rows directly.  (Causal, such a block sees 32 keys at most;
+        // below 256 keys the prefill body starts faster: 256 x 16 x 64
         // 5.1 against 5.9 us.)  Measured on MI355X against the key-split
         // prefill, bf16, us: 32 x 16 x 32768 d128 101.8 -> 83.2, 256 x 16 x
         // 8192 186 -> 153 (7.0 TB/s), d64 114 -> 77, d256 32 x 16 x 32768 184
@@ -435,7 +435,12 @@ int make_plan(int variant, const void* q, const void* k, const void* v, const fl
             size_t len = ((sk + n - 1) / n + 63) / 64 * 64;
             n = (sk + len - 1) / len;
             if (n <= (size_t)kMaxSplits && len <= imax && bh * n <= imax && bh * sq <= imax) {
-                plan->first.name += "s";
+                if (D == 128) {
+                    plan->first.name += "s";
+                } else {
+                    std::snprintf(buf, sizeof(buf), "fa_prefill_lp_%s_d%d_2_rows", dtype == FA_DTYPE_BF16 ? "bf16" : "f16", D);
+                    plan->first.name = buf;
+                }
                 plan->first.gx = static_cast<unsigned>(bh * n);
                 plan->first.bx = 64 * fa_lp_waves(lp_tiles);
                 p.few_rows = 1;
@@ -565,13 +570,17 @@ int make_plan(int variant, const void* q, const void* k, const void* v, const fl
                 // (MI355X, bf16; every shape of 1 .. 32 heads x 512 .. 4096
                 // within 15 %), fixed + per 64 keys: the plain kernel; 64, 96 or
                 // 128 rows with 4, 2, 2 waves on each tile's keys (D = 64, 128;
+                // at D = 256, whose registers allow 8 waves, 64 with 2;
                 // causal: folded), where they all run at once; the key split,
                 // whose kernel is slower a stage (its segment loop) and which
                 // adds a merge launch and its partials, written and read back
-                // at 4 TB/s.  us before -> now: 16 x 1500^2 d64 36.9 -> 17.7 (96
+                // at 4 TB/s (at D = 256 and one workgroup per CU 9 us at most:
+                // 80 .. 256 workgroups, 11 .. 14 us with the merge launch).  us before -> now: 16 x 1500^2 d64 36.9 -> 17.7 (96
                 // rows; key split before), 16 x 1024^2 23.8 -> 11.3 and d128 36.5
                 // -> 16.4 (64), causal 8 x 2048^2 33.4 -> 24.1 (64), 16 x 2048^2
-                // 41.2 -> 30.1 and 8 x 4096^2 75.4 -> 50.0 (128; plain before).
+                // 41.2 -> 30.1 and 8 x 4096^2 75.4 -> 50.0 (128; plain before);
+                // d256 16 x 1024^2 38.0 -> 27.6 (plain before), 8 x 2048^2 53.4
+                // -> 45.8 (key split before).
                 // The key split stays for few blocks of many keys: 1 x 2048^2
                 // d64 13.9 against 17.2.
                 const double cus = (double)num_cus, keys = (double)max_st;
@@ -583,11 +592,13 @@ int make_plan(int variant, const void* q, const void* k, const void* v, const fl
                 size_t wide = 0, wide_blocks = 0;   // rows and blocks (pairs of half blocks) per slice
                 bool wide_fold = false;
                 // (up to 128 keys a block has two stages)
-                if ((D == 64 || D == 128) && sk > 128) {
-                    const struct { size_t rows; double fixed, key64, causal64; } form[2][3] = {
+                if (D >= 64 && sk > 128) {
+                    const struct { size_t rows; double fixed, key64, causal64; } form[3][3] = {
                         {{64, 4.8, 0.385, 0.37}, {96, 5.0, 0.50, 0.40}, {128, 5.0, 0.62, 0.43}},
-                        {{64, 6.6, 0.54, 0.51}, {96, 6.7, 0.72, 0.57}, {128, 6.5, 0.90, 0.62}}};
-                    for (const auto& f : form[D == 128]) {
+                        {{64, 6.6, 0.54, 0.51}, {96, 6.7, 0.72, 0.57}, {128, 6.5, 0.90, 0.62}},
+                        {{64, 7.0, 1.20, 1.16}}};
+                    for (const auto& f : form[D == 64 ? 0 : D == 128 ? 1 : 2]) {
+                        if (!f.rows) break;
                         const size_t half = f.rows / 2, nhb = (sq + half - 1) / half;
                         const bool fold = causal && nhb >= 2;
                         const size_t nb = (nhb + 1) / 2;
@@ -614,7 +625,9 @@ int make_plan(int variant, const void* q, const void* k, const void* v, const fl
                     const double n = (double)wgs_for(lo);
                     // two workgroups on a CU (D <= 128) take 1.5 times one's time
                     const double turns = D <= 128 ? (n <= cus ? 1.0 : 1.5 * std::ceil(n / (2.0 * cus))) : std::ceil(n / cus);
-                    const double t = turns * (fix + split * (double)lo) + 5.5 + n * 128.0 * (4.0 * D + 8.0) * 2.0 / 4.0e6;
+                    double part = n * 128.0 * (4.0 * D + 8.0) * 2.0 / 4.0e6;
+                    if (D == 256 && n <= cus) part = std::min(part, 9.0);
+                    const double t = turns * (fix + split * (double)lo) + 5.5 + part;
                     if (t < best) {
                         best = t;
                         per = lo;
@@ -626,7 +639,7 @@ int make_plan(int variant, const void* q, const void* k, const void* v, const fl
                                   static_cast<int>(wide));
                     plan->first.name = buf;
                     plan->first.gx = static_cast<unsigned>(wide_blocks * bh);
-                    plan->first.bx = wide == 96 ? 768 : 1024;
+                    plan->first.bx = D == 256 ? 512 : wide == 96 ? 768 : 1024;
                     p.nqb = static_cast<int>(wide_blocks);
                     p.fold = wide_fold ? 1 : 0;
                     p.pair_w = 0;

@@ -10,7 +10,9 @@
 //   pv4 / axpy / scale_inplace  -> PV on v_mfma_f32_16x16x4_f32, per-lane rescale
 //   naive_attention src/naive.rs:14-75 -> naive_{scores,softmax,pv}_body
 //   (new) split-KV + LSE merge  -> decode_body / merge_body (short queries,
-//                                  and the prefill key split on small grids)
+//                                  and the prefill key and stream splits)
+//   (new) small f32 grids       -> prefill_fold_body (fa_fold.inc, v2 and v3)
+//   (new) 16-bit inputs         -> fa_lp.inc
 //
 // All arithmetic is IEEE f32 (f32 MFMA, no reduced-precision inputs); the
 // naive kernels also have an f64 instantiation for on-device checking.
@@ -18,7 +20,8 @@
 // Prefill geometry (D = d_head padded to 32/64/128/256/512/1024; fa_params.h):
 //   * a workgroup of NW = 8 waves owns BQ = 128 query rows of one
 //     (batch*head) slice; wave w owns rows 16w .. 16w+15 (D > 256: column
-//     groups of D/256 waves share a 16-row tile, 256 columns each);
+//     groups of D/256 waves share a 16-row tile, 256 columns each); a folded
+//     causal grid takes 64 rows from each end of the slice (p.fold);
 //   * keys stream through LDS in stages of SK keys (64 for D <= 128, 32 or
 //     16 for D = 256), K rows padded to D+8 floats and V rows to D+16 (D+8
 //     at D = 32) so 128-bit reads are free of bank conflicts on the 128-bank

@@ -35,7 +35,7 @@ typedef struct FaParams {
     int fold;            // f32 v2 / v3 prefill, causal: a workgroup's lower 64 rows are half block
                          // nhb-1-r of the slice, its upper 64 rows half block r (equal work per
                          // workgroup); 0 = 128 consecutive rows
-    int few_rows;        // 16-bit split kernels: at most 32 query rows, num_splits workgroups per slice
+    int few_rows;        // 16-bit D = 128 split kernel: at most 32 query rows, num_splits workgroups per slice
                          // stream split_len keys each
     int full_keys;       // v1: every query block visits all seq_k keys, causal or not (no
                          // causal skip), so the key split, the stream split and fa_merge

@@ -61,6 +61,8 @@ def test_few_rows_are_planned_only_for_their_calls():
     assert s.startswith("fa_prefill_lp_bf16_d128_2_t2s grid=256x1x1 block=256; fa_merge_d128 grid=128x1x1")
     assert "splits=8 split_len=4096" in s
     assert "splits=32 split_len=256" in plan(1, 8, 8192, 64, False)
+    assert plan(256, 16, 8192, 256, False) == "fa_prefill_lp_bf16_d256_2_rows grid=256x1x1 block=512"
+    assert plan(256, 32, 8192, 64, False) == "fa_prefill_lp_bf16_d64_2_rows grid=256x1x1 block=512"
     for other in (plan(256, 33, 8192, 128, False), plan(256, 17, 8192, 256, False),   # rows
                   plan(256, 16, 8192, 128, True), plan(256, 16, 255, 128, False),     # causal, few keys
                   plan(256, 16, 8192, 100, False), plan(256, 16, 8192, 32, False)):   # scalar loads, D = 32

@@ -1,7 +1,7 @@
 """16-bit prefills of at most one 128-row block per CU: workgroups of 64, 96 or
-128 rows with 4, 2 and 2 waves on each 16-row tile's keys, causal ones folded
-(rows from both ends of the slice).  At the edges of half blocks, stages of 128
-keys and the waves' shares of them.  Against float64 attention on the same
+128 rows with 4, 2 and 2 waves on each 16-row tile's keys (D = 256: 64 with 2),
+causal ones folded (rows from both ends of the slice).  At the edges of half
+blocks, stages of 128 keys (D = 256: 64) and the waves' shares of them.  Against float64 attention on the same
 16-bit inputs under the 16-bit path's derived bound (probabilities rounded
 once: u / (1 - u) max|V|, u = 2^-8 bf16, 2^-11 f16, plus 2e-5 for the f32
 sums)."""
@@ -29,6 +29,11 @@ SHAPES = [
     (128, 64, 449, 449, 64, True),    # 8 half blocks of 64 rows, one row in the last
     (128, 84, 300, 300, 128, True),   # 5: the middle one alone
     (128, 64, 400, 321, 72, False),   # the second waves have one key of the last stage
+    (64, 3, 129, 129, 256, True),     # stages of 64 keys: 5 half blocks, the middle one alone, one key in the third
+    (64, 8, 289, 289, 200, True),     # 10, one row in the last, d < D
+    (64, 3, 300, 777, 256, False),
+    (64, 2, 700, 300, 256, True),
+    (64, 8, 130, 161, 136, False),    # the second waves have one key of the last stage
 ]
 
 
@@ -48,7 +53,7 @@ def test_shared_tiles(shape, name):
     rows, bh, sq, sk, d, causal = shape
     dt, u = DT[name]
     plan = fa.describe_launch(2, 1, bh, sq, sk, d, causal, dtype=dt)
-    assert plan.startswith(f"fa_prefill_lp_{name}_d{64 if d <= 64 else 128}_2_t1r{rows} "), plan
+    assert plan.startswith(f"fa_prefill_lp_{name}_d{64 if d <= 64 else 128 if d <= 128 else 256}_2_t1r{rows} "), plan
     q, qf = inputs(name, bh * sq * d, 1)
     k, kf = inputs(name, bh * sk * d, 2)
     v, vf = inputs(name, bh * sk * d, 3)
@@ -68,9 +73,10 @@ def test_shared_tiles_are_planned_only_for_their_calls():
     assert "t1r96 grid=256x1x1 block=768" in plan(16, 1500, 1500, 64, False)
     assert "t1r128 grid=256x1x1 block=1024" in plan(16, 2048, 2048, 128, True)
     assert "t1r64 grid=256x1x1 block=1024" in plan(8, 2048, 2048, 64, True)
+    assert "t1r64 grid=256x1x1 block=512" in plan(16, 1024, 1024, 256, False)
     for other in (plan(17, 2048, 2048, 128, True), plan(32, 2048, 2048, 128, True),   # more blocks than CUs
                   plan(8, 128, 128, 64, True), plan(8, 1000, 1000, 62, True),         # few keys, scalar loads
-                  plan(8, 1000, 1000, 256, True), plan(8, 1000, 1000, 32, True),
+                  plan(8, 1000, 1000, 32, True), plan(16, 2048, 2048, 256, True),
                   plan(8, 1000, 1000, 64, True, path=fa.PATH_PREFILL), plan(8, 1000, 1000, 64, True, path=fa.PATH_STREAM),
                   plan(1, 4096, 4096, 128, True)):                                    # few blocks of many keys: key split
         assert "t1r" not in other, other
