@@ -751,7 +751,17 @@ int make_plan(int variant, const void* q, const void* k, const void* v, const fl
                 p.two_blocks = 1;
                 plan->first.gx = static_cast<unsigned>(nqb / 2 * bh);
             }
-            if (per == 0 && fold_ok && path == FA_PATH_AUTO && !p.two_blocks) p.fold = 1;
+            if (per == 0 && fold_ok && path == FA_PATH_AUTO && !p.two_blocks) {
+                p.fold = 1;
+                // v2's folded grids run v3's kernel where it has the DMA: same
+                // sums, the next stage's QK^T among this one's PV.  us: 16 x
+                // 2048^2 d64 84.0 -> 78.7, d128 159.8 -> 143.9, d256 331 -> 298,
+                // 32 x 1024^2 d256 176 -> 159, 16 x 2048^2 d32 48.3 -> 47.6.
+                if (variant == 2 && vec) {
+                    std::snprintf(buf, sizeof(buf), "fa_prefill_v3_d%d_2", D);
+                    plan->first.name = buf;
+                }
+            }
             if (per > 0) {
                 const size_t nks = (max_st + per - 1) / per;
                 if (nks > 65535 || nks > (size_t)kMaxSplits) return FA_ERR_UNSUPPORTED;
