@@ -622,6 +622,11 @@ int make_plan(int variant, const void* q, const void* k, const void* v, const fl
                         else lo = mid + 1;
                     }
                     if ((max_st + lo - 1) / lo < 2) continue;
+                    // A grid of one block per CU needs no workspace unsplit, so it
+                    // is split only within the allocation-free form's scratch.
+                    if (nqb * bh == (size_t)num_cus &&
+                        bh * nqt * ((max_st + lo - 1) / lo) * (16 * (size_t)D + 32) * sizeof(float) > FA_SCRATCH_BYTES)
+                        continue;
                     const double n = (double)wgs_for(lo);
                     // two workgroups on a CU (D <= 128) take 1.5 times one's time
                     const double turns = D <= 128 ? (n <= cus ? 1.0 : 1.5 * std::ceil(n / (2.0 * cus))) : std::ceil(n / cus);

@@ -74,6 +74,8 @@ def test_shared_tiles_are_planned_only_for_their_calls():
     assert "t1r128 grid=256x1x1 block=1024" in plan(16, 2048, 2048, 128, True)
     assert "t1r64 grid=256x1x1 block=1024" in plan(8, 2048, 2048, 64, True)
     assert "t1r64 grid=256x1x1 block=512" in plan(16, 1024, 1024, 256, False)
+    # one block per CU: no split whose partials pass the 64 MiB of the allocation-free form
+    assert plan(4, 8192, 8192, 256, True) == "fa_prefill_lp_bf16_d256_2_t1 grid=256x1x1 block=512"
     for other in (plan(17, 2048, 2048, 128, True), plan(32, 2048, 2048, 128, True),   # more blocks than CUs
                   plan(8, 128, 128, 64, True), plan(8, 1000, 1000, 62, True),         # few keys, scalar loads
                   plan(8, 1000, 1000, 32, True), plan(16, 2048, 2048, 256, True),
