@@ -426,15 +426,20 @@ int make_plan(int variant, const void* q, const void* k, const void* v, const fl
         // prefill, bf16, us: 32 x 16 x 32768 d128 101.8 -> 83.2, 256 x 16 x
         // 8192 186 -> 153 (7.0 TB/s), d64 114 -> 77, d256 32 x 16 x 32768 184
         // -> 160; two workgroups per CU 83.8 / 161 / 84 / 187.  Two short
-        // splits lose to one: 128 x 16 x 1024 16.7 against 14.9.
+        // splits lose to one: 128 x 16 x 1024 16.7 against 14.9; with two
+        // tiles or at D = 256 that one loses to the small grids' workgroups
+        // below (64 x 32 x 674 15.7 against 11.5, 128 x 2 x 1630 d256 42.2
+        // against 37.0).
         const size_t few = D <= 128 ? 32 : 16;
         if (lp && path == FA_PATH_AUTO && vec && D >= 64 && !causal && sq <= few && sk >= kMinSplitKeys) {
             size_t n = std::max<size_t>(1, (size_t)num_cus / bh);
             n = std::min(n, std::max<size_t>(1, sk / kMinSplitKeys));
-            if (n == 2 && sk < 2048) n = 1;
+            const bool short2 = n == 2 && sk < 2048;
+            if (short2) n = 1;
             size_t len = ((sk + n - 1) / n + 63) / 64 * 64;
             n = (sk + len - 1) / len;
-            if (n <= (size_t)kMaxSplits && len <= imax && bh * n <= imax && bh * sq <= imax) {
+            if (n <= (size_t)kMaxSplits && len <= imax && bh * n <= imax && bh * sq <= imax &&
+                !(short2 && (sq > 16 || D == 256))) {
                 if (D == 128) {
                     plan->first.name += "s";
                 } else {
@@ -591,8 +596,10 @@ int make_plan(int variant, const void* q, const void* k, const void* v, const fl
                 best = fix + plain * keys;
                 size_t wide = 0, wide_blocks = 0;   // rows and blocks (pairs of half blocks) per slice
                 bool wide_fold = false;
-                // (up to 128 keys a block has two stages)
-                if (D >= 64 && sk > 128) {
+                // (up to 128 keys a block has two stages; causal, up to three the
+                // plain kernel is the faster: 40 x 188^2 d128 7.8 against 8.8
+                // us, 4 x 256^2 9.4 against 8.6)
+                if (D >= 64 && sk > (causal && D <= 128 ? 208u : 128u)) {
                     const struct { size_t rows; double fixed, key64, causal64; } form[3][3] = {
                         {{64, 4.8, 0.385, 0.37}, {96, 5.0, 0.50, 0.40}, {128, 5.0, 0.62, 0.43}},
                         {{64, 6.6, 0.54, 0.51}, {96, 6.7, 0.72, 0.57}, {128, 6.5, 0.90, 0.62}},
@@ -628,8 +635,12 @@ int make_plan(int variant, const void* q, const void* k, const void* v, const fl
                         bh * nqt * ((max_st + lo - 1) / lo) * (16 * (size_t)D + 32) * sizeof(float) > FA_SCRATCH_BYTES)
                         continue;
                     const double n = (double)wgs_for(lo);
-                    // two workgroups on a CU (D <= 128) take 1.5 times one's time
-                    const double turns = D <= 128 ? (n <= cus ? 1.0 : 1.5 * std::ceil(n / (2.0 * cus))) : std::ceil(n / cus);
+                    // two workgroups on a CU (D <= 128) take 1.35 times one's time,
+                    // those of the two-tile kernel (a wave per SIMD each) the same
+                    // (bf16 d128, us, before -> now: 2 x 6000^2 60.3 -> 52.0,
+                    // 1 x 8000^2 56.3 -> 47.8; d32 256 x 16 x 8192 87.1 -> 74.2)
+                    const double pair = two ? 1.0 : 1.35;
+                    const double turns = D <= 128 ? (n <= cus ? 1.0 : pair * std::ceil(n / (2.0 * cus))) : std::ceil(n / cus);
                     double part = n * 128.0 * (4.0 * D + 8.0) * 2.0 / 4.0e6;
                     if (D == 256 && n <= cus) part = std::min(part, 9.0);
                     const double t = turns * (fix + split * (double)lo) + 5.5 + part;
@@ -655,7 +666,9 @@ int make_plan(int variant, const void* q, const void* k, const void* v, const fl
                 // no split: the longest block, or with the folded grid half
                 // the keys of its long and its short half block together
                 best = std::ceil((double)(nqb * bh) / cus) * (double)max_st * skd;
-                if (fold_ok) best = fold_keys(rows / 2);
+                // (8 % slower a key at D = 256: 12 x 2368^2 340 us folded, 325 on
+                // the stream split)
+                if (fold_ok) best = (D == 256 ? 1.08 : 1.0) * fold_keys(rows / 2);
                 // Candidates: for R = 1..4 rounds, the shortest split whose
                 // workgroups fit in R rounds (workgroup count falls as `per`
                 // grows, so bisect).

@@ -65,5 +65,5 @@ def test_few_rows_are_planned_only_for_their_calls():
     assert plan(256, 32, 8192, 64, False) == "fa_prefill_lp_bf16_d64_2_rows grid=256x1x1 block=512"
     for other in (plan(256, 33, 8192, 128, False), plan(256, 17, 8192, 256, False),   # rows
                   plan(256, 16, 8192, 128, True), plan(256, 16, 255, 128, False),     # causal, few keys
-                  plan(256, 16, 8192, 100, False), plan(256, 16, 8192, 32, False)):   # scalar loads, D = 32
+                  plan(256, 16, 8192, 100, False), plan(256, 16, 4096, 32, False)):   # scalar loads, D = 32
         assert not other.split()[0].endswith("s"), other
