@@ -124,8 +124,8 @@ int fa_attention_multihead(const float* q, size_t q_len, const float* k, size_t 
  * default stream).  No length checks are possible on raw pointers; zero
  * dims return FA_OK with nothing queued.  Every variant picks the split-KV
  * (flash-decoding) kernels for short query blocks against long key ranges,
- * and a key or stream split on grids smaller than the GPU (v1 on kernels of
- * its own that keep its per-step normalisation and visit every key, causal
+ * and smaller workgroups (v2, v3) or a key or stream split on grids smaller
+ * than the GPU (v1 on kernels of its own that keep its per-step normalisation and visit every key, causal
  * or not).  Their partials go to a
  * workspace kept per stream (up to 256 MiB; larger ones are allocated and
  * released stream-ordered around the call): the first call on a stream that
@@ -174,8 +174,10 @@ int fa_release_stream_workspace(void* stream);
  * normalisation and visit every key (no causal skip).  AUTO runs
  * decode steps -- seq_len_q <= 32, any batch and key count -- on split-KV
  * (the row-streaming kernel where it applies, else 16-row tiles; 16-bit
- * inputs only on the row kernel), and the stream split or the key split for
- * prefills smaller than the GPU.
+ * inputs on the row kernel for one query, on a streaming prefill kernel for
+ * more), and prefills smaller than the GPU on smaller workgroups whose waves
+ * share the keys of a query tile, on the stream split or on the key split,
+ * whichever it estimates to be fastest.
  * num_splits = 0 lets the library choose (at most 1024). */
 #define FA_PATH_AUTO 0
 #define FA_PATH_PREFILL 1
