@@ -419,8 +419,8 @@ __device__ __forceinline__ void prefill_segment(const FaParams& p, const Prefill
     // long tile and one short one, and once the short tile is through, the
     // long one has the SIMD to itself (f32 MFMAs hold the SIMD: a lone wave's
     // stage takes 0.52 of two waves').  v3 16 x 2048^2: d128 247 -> 144 us,
-    // d64 130 -> 79.
-    const bool fold = !STREAM && VARIANT != 1 && CG == 1 && p.fold != 0;
+    // d64 130 -> 79.  (v2's folded grids with 128-bit operands run v3's kernel.)
+    const bool fold = !STREAM && VARIANT != 1 && !(VARIANT == 2 && LOADER == 1) && CG == 1 && p.fold != 0;
     const int nhb = (seq_q + BQ / 2 - 1) / (BQ / 2);
     const int row_a = !fold ? q0 + 16 * tile
                       : tile < TILES / 2 ? (nhb - 1 - qb) * (BQ / 2) + 16 * tile
