@@ -618,7 +618,7 @@ int make_plan(int variant, const void* q, const void* k, const void* v, const fl
                         }
                     }
                 }
-                for (size_t R = 1; R <= 4; ++R) {
+                for (size_t R = 1; R <= 4 && nqb * bh < (size_t)num_cus; ++R) {
                     // the shortest split whose workgroups fit R per CU
                     const size_t slots = R * (size_t)num_cus;
                     size_t lo = 4, hi = max_st;
@@ -629,16 +629,17 @@ int make_plan(int variant, const void* q, const void* k, const void* v, const fl
                         else lo = mid + 1;
                     }
                     if ((max_st + lo - 1) / lo < 2) continue;
-                    // A grid of one block per CU needs no workspace unsplit, so it
-                    // is split only within the allocation-free form's scratch.
-                    if (nqb * bh == (size_t)num_cus &&
-                        bh * nqt * ((max_st + lo - 1) / lo) * (16 * (size_t)D + 32) * sizeof(float) > FA_SCRATCH_BYTES)
-                        continue;
                     const double n = (double)wgs_for(lo);
+                    // Nearly full grids stay unsplit: the rounds of one workgroup
+                    // per CU have to be fewer than the splits, so that a call that
+                    // can run without a workspace (captured on any stream,
+                    // overlapping others in the allocation-free form) does.
+                    if (std::ceil(n / cus) * ((double)(lo * SKs) + kOverheadKeys) + n / cus * kOverheadKeys >= keys * (double)SKs)
+                        continue;
                     // two workgroups on a CU (D <= 128) take 1.35 times one's time,
                     // those of the two-tile kernel (a wave per SIMD each) the same
                     // (bf16 d128, us, before -> now: 2 x 6000^2 60.3 -> 52.0,
-                    // 1 x 8000^2 56.3 -> 47.8; d32 256 x 16 x 8192 87.1 -> 74.2)
+                    // 1 x 8000^2 56.3 -> 47.8)
                     const double pair = two ? 1.0 : 1.35;
                     const double turns = D <= 128 ? (n <= cus ? 1.0 : pair * std::ceil(n / (2.0 * cus))) : std::ceil(n / cus);
                     double part = n * 128.0 * (4.0 * D + 8.0) * 2.0 / 4.0e6;

@@ -82,3 +82,14 @@ def test_shared_tiles_are_planned_only_for_their_calls():
                   plan(8, 1000, 1000, 64, True, path=fa.PATH_PREFILL), plan(8, 1000, 1000, 64, True, path=fa.PATH_STREAM),
                   plan(1, 4096, 4096, 128, True)):                                    # few blocks of many keys: key split
         assert "t1r" not in other, other
+
+
+def test_nearly_full_grids_need_no_workspace():
+    """Non-causal grids that leave less than a fifth of the CUs idle run unsplit:
+    without a workspace they can be captured on any stream and may overlap
+    other calls of the allocation-free form."""
+    for bh, sq, sk, d in ((3, 9865, 9865, 128), (2, 13956, 13956, 96), (3, 8930, 31345, 96), (5, 5821, 5821, 32),
+                          (236, 10, 29259, 32), (256, 16, 8192, 32), (237, 32, 7001, 32), (2, 16384, 16384, 64)):
+        for name in DT:
+            plan = fa.describe_launch(2, 1, bh, sq, sk, d, False, dtype=DT[name][0])
+            assert "workspace" not in plan, (bh, sq, sk, d, plan)
