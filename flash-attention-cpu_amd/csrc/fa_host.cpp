@@ -618,6 +618,12 @@ int make_plan(int variant, const void* q, const void* k, const void* v, const fl
                         }
                     }
                 }
+                // Nearly full grids (more than 4/5 of the CUs, non-causal) stay
+                // unsplit: with one workgroup per CU no number of rounds would be
+                // smaller than its number of splits, and a call that can run
+                // without a workspace (captured on any stream, overlapping others
+                // in the allocation-free form) does.
+                bool uneven = false;
                 for (size_t R = 1; R <= 4 && nqb * bh < (size_t)num_cus; ++R) {
                     // the shortest split whose workgroups fit R per CU
                     const size_t slots = R * (size_t)num_cus;
@@ -630,12 +636,8 @@ int make_plan(int variant, const void* q, const void* k, const void* v, const fl
                     }
                     if ((max_st + lo - 1) / lo < 2) continue;
                     const double n = (double)wgs_for(lo);
-                    // Nearly full grids stay unsplit: the rounds of one workgroup
-                    // per CU have to be fewer than the splits, so that a call that
-                    // can run without a workspace (captured on any stream,
-                    // overlapping others in the allocation-free form) does.
-                    if (std::ceil(n / cus) * ((double)(lo * SKs) + kOverheadKeys) + n / cus * kOverheadKeys >= keys * (double)SKs)
-                        continue;
+                    if (std::ceil(n / cus) * ((double)(lo * SKs) + kOverheadKeys) + n / cus * kOverheadKeys < keys * (double)SKs)
+                        uneven = true;
                     // two workgroups on a CU (D <= 128) take 1.35 times one's time,
                     // those of the two-tile kernel (a wave per SIMD each) the same
                     // (bf16 d128, us, before -> now: 2 x 6000^2 60.3 -> 52.0,
@@ -648,9 +650,10 @@ int make_plan(int variant, const void* q, const void* k, const void* v, const fl
                     if (t < best) {
                         best = t;
                         per = lo;
-                        wide = 0;
                     }
                 }
+                if (!uneven) per = 0;
+                if (per > 0) wide = 0;
                 if (wide) {
                     std::snprintf(buf, sizeof(buf), "fa_prefill_lp_%s_d%d_2_t1r%d", dtype == FA_DTYPE_BF16 ? "bf16" : "f16", D,
                                   static_cast<int>(wide));

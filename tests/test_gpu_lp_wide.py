@@ -93,3 +93,5 @@ def test_nearly_full_grids_need_no_workspace():
         for name in DT:
             plan = fa.describe_launch(2, 1, bh, sq, sk, d, False, dtype=DT[name][0])
             assert "workspace" not in plan, (bh, sq, sk, d, plan)
+    # from 4/5 of the CUs down a split is taken where it is the faster: two splits, 27 MB
+    assert "splits=2 " in fa.describe_launch(2, 1, 204, 119, 10566, 128, False, dtype=fa.DTYPE_BF16)
