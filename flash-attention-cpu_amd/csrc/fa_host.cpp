@@ -654,6 +654,29 @@ int make_plan(int variant, const void* q, const void* k, const void* v, const fl
                 }
                 if (!uneven) per = 0;
                 if (per > 0) wide = 0;
+                // Causal, few keys on a nearly full grid: what the estimates above
+                // leave out decides between the small workgroups (128 rows, 96
+                // at D = 128) and the plain kernel -- the bytes of the first
+                // fetches and last stores (per MB of Q, K, V and O) and, with
+                // fewer keys than queries, the keys that both half blocks of a
+                // pair see.  Fitted to 440 shapes (3 .. 7 % rms).  Plain against
+                // the workgroups that the estimates above take, us: 114 x 210^2
+                // d128 10.2 / 12.3, 93 x 226^2 10.2 / 11.9, 43 x 604 x 243 12.1 /
+                // 13.9, 91 x 204 x 1712 d64 6.9 / 8.0; the workgroups stay from
+                // about 700 keys on at D = 128 and 500 at 64.  (64 rows, and 96 at
+                // D = 64, stay: 0.93 .. 1.0 of plain from 208 keys on.)
+                if (causal && (wide == 128 || (wide == 96 && D == 128))) {
+                    const struct { double fixed, both64, long64, mb; } us[3] = {{4.9, 0.62, 0.425, 0.08}, {5.5, 0.78, 0.61, 0.10}, {6.0, 0.95, 0.63, 0.12}};
+                    const auto& f = us[D == 64 ? 0 : wide == 96 ? 1 : 2];
+                    const size_t half = wide / 2, nhb = (sq + half - 1) / half;
+                    const double end = (double)std::min(sk, nhb * half);                       // longest pair's
+                    const double mid = (double)std::min(sk, ((nhb - 1) / 2 + 1) * half);       // middle pair's short half
+                    const double mb = (double)bh * (double)d * 1e-6 *
+                                      (6.0 * (double)sq + 4.0 * (double)std::min(sk, nqb * rows));
+                    const double t = f.fixed + f.mb * mb + (f.long64 * end + std::max(0.0, f.both64 - f.long64) *
+                                                                                   std::max(0.0, 2.0 * mid - end)) / 64.0;
+                    if (t >= (D == 128 ? 3.5 + 1.09 * keys + 0.08 * mb : 3.2 + 0.80 * keys + 0.065 * mb)) wide = 0;
+                }
                 if (wide) {
                     std::snprintf(buf, sizeof(buf), "fa_prefill_lp_%s_d%d_2_t1r%d", dtype == FA_DTYPE_BF16 ? "bf16" : "f16", D,
                                   static_cast<int>(wide));

@@ -24,10 +24,10 @@ SHAPES = [
     (64, 4, 129, 513, 128, False),    # one row in the third block, one key in the fifth stage
     (64, 4, 100, 577, 64, False),     # the waves' shares of the last stage: 32, 32, 1 and no keys
     (96, 64, 300, 300, 64, True),     # 7 half blocks of 48 rows: the middle one alone
-    (96, 64, 289, 289, 128, True),    # 7, one row in the last
+    (96, 56, 337, 337, 128, True),    # 8, one row in the last
     (96, 64, 300, 193, 128, False),
     (128, 64, 449, 449, 64, True),    # 8 half blocks of 64 rows, one row in the last
-    (128, 84, 300, 300, 128, True),   # 5: the middle one alone
+    (128, 40, 690, 690, 128, True),   # 11: the middle one alone
     (128, 64, 400, 321, 72, False),   # the second waves have one key of the last stage
     (64, 3, 129, 129, 256, True),     # stages of 64 keys: 5 half blocks, the middle one alone, one key in the third
     (64, 8, 289, 289, 200, True),     # 10, one row in the last, d < D
@@ -95,3 +95,16 @@ def test_nearly_full_grids_need_no_workspace():
             assert "workspace" not in plan, (bh, sq, sk, d, plan)
     # from 4/5 of the CUs down a split is taken where it is the faster: two splits, 27 MB
     assert "splits=2 " in fa.describe_launch(2, 1, 204, 119, 10566, 128, False, dtype=fa.DTYPE_BF16)
+
+
+def test_short_causal_calls_keep_the_plain_kernel():
+    """Causal calls of few keys on a nearly full grid, measured slower on the
+    small workgroups (bf16, us: plain, small)."""
+    for bh, sq, sk, d in ((114, 210, 210, 128),     # 10.2, 12.3
+                          (93, 226, 226, 128),      # 10.2, 11.9
+                          (43, 604, 243, 128),      # 12.1, 13.9
+                          (53, 397, 397, 128),      # 13.5, 14.5
+                          (91, 204, 1712, 64),      # 6.9, 8.0
+                          (4, 6159, 255, 64)):      # 7.7, 8.5
+        plan = fa.describe_launch(2, 1, bh, sq, sk, d, True, dtype=fa.DTYPE_BF16)
+        assert "_t1 " in plan, (bh, sq, sk, d, plan)
