@@ -490,7 +490,7 @@ int make_plan(int variant, const void* q, const void* k, const void* v, const fl
         // (map_block), and folding would make its last round a full one.
         // Measured on MI355X (v3, causal): 16 x 2048^2 d128 247 -> 148 us,
         // 32 x 1024^2 d128 126 -> 81, 16 x 2048^2 d64 130 -> 79.
-        const bool fold_ok = !lp && causal_skip && D <= kMaxDNarrow && nqb >= 2 && nqb * bh <= (size_t)num_cus;
+        bool fold_ok = !lp && causal_skip && D <= kMaxDNarrow && nqb >= 2 && nqb * bh <= (size_t)num_cus;
         // f32 v3 with 128-bit DMA and d = D = 128: pair query blocks nqb-1-r
         // and r in one workgroup (equal causal work per workgroup; the
         // second block's loads overlap the first's last step) when the
@@ -690,12 +690,8 @@ int make_plan(int variant, const void* q, const void* k, const void* v, const fl
                 }
             } else if (path == FA_PATH_AUTO && nqb * bh < (size_t)num_cus) {
                 const double cus = (double)num_cus, skd = (double)SKs;
-                // no split: the longest block, or with the folded grid half
-                // the keys of its long and its short half block together
+                // no split: the longest block
                 best = std::ceil((double)(nqb * bh) / cus) * (double)max_st * skd;
-                // (8 % slower a key at D = 256: 12 x 2368^2 340 us folded, 325 on
-                // the stream split)
-                if (fold_ok) best = (D == 256 ? 1.08 : 1.0) * fold_keys(rows / 2);
                 // Candidates: for R = 1..4 rounds, the shortest split whose
                 // workgroups fit in R rounds (workgroup count falls as `per`
                 // grows, so bisect).
@@ -726,6 +722,40 @@ int make_plan(int variant, const void* q, const void* k, const void* v, const fl
                         stream = true;
                     }
                 }
+            }
+            // The folded grid in place of a split: half the keys of its long and
+            // its short half block together have to be fewer than the split's
+            // cost (8 % slower a key at D = 256: 12 x 2368^2 340 us folded, 325 on
+            // the stream split), and its time, in us, fixed + per key of those
+            // costs, the shorter one.  Fitted to 207 causal f32 calls (v2 and
+            // v3; 2 .. 8 % rms); by keys alone it had been taken for, us, 41 x
+            // 273^2 d256 59.5 (key split 53.8), 48 x 220 x 2808 d200 49.5 (40.9),
+            // 26 x 811 x 933 d160 128.9 (stream split 119.5), 2 x 8350 x 391 d128
+            // 61.3 (52.4), 20 x 922^2 d72 71.2 (64.5).  No split past the
+            // allocation-free form's scratch takes its place.
+            const bool cut = per > 0 && (max_st + per - 1) / per >= 2;
+            if (fold_ok && path == FA_PATH_AUTO && (stream || cut)) {
+                static constexpr struct { double fixed, key; } us[4][3] = {   // folded, key split, stream split
+                    {{4.0, 0.0390}, {6.7, 0.0417}, {12.9, 0.0387}},      // D = 32
+                    {{5.0, 0.0670}, {1.1, 0.0762}, {4.6, 0.0678}},       // 64
+                    {{8.5, 0.1256}, {-0.3, 0.134}, {-2.7, 0.1326}},      // 128
+                    {{7.0, 0.267}, {-8.8, 0.2807}, {-16.2, 0.2763}}};    // 256
+                const double keys = (D == 256 ? 1.08 : 1.0) * fold_keys(rows / 2);
+                // the longest pair of two half blocks (an odd count's middle one has a SIMD alone)
+                const size_t half = rows / 2, nhb = (sq + half - 1) / half, r = nhb / 2 - 1;
+                const double pair = 0.5 * (double)(std::min(sk, (nhb - r) * half) + std::min(sk, (r + 1) * half));
+                const auto* u = us[D == 32 ? 0 : D == 64 ? 1 : D == 128 ? 2 : 3];
+                const auto& o = u[stream ? 2 : 1];
+                const size_t tiles = stream ? (s_wgs + bh * nqb - 1) * (rows / 16) : bh * nqt * ((max_st + per - 1) / per);
+                const bool large = tiles * (16 * (size_t)D + 32) * sizeof(float) > FA_SCRATCH_BYTES;
+                fold_ok = keys <= best && (large || u[0].fixed + u[0].key * pair <= o.fixed + o.key * best);
+                if (fold_ok) {
+                    best = keys;
+                    per = 0;
+                    stream = false;
+                }
+            } else if (fold_ok && path == FA_PATH_AUTO) {
+                best = (D == 256 ? 1.08 : 1.0) * fold_keys(rows / 2);
             }
             // Smaller workgroups (fa_fold.inc): 8 / G tiles of 16 rows, G
             // waves sharing a tile's keys, no workspace and no merge launch.

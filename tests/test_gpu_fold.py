@@ -105,3 +105,17 @@ def test_shared_tiles_are_planned_only_for_their_calls():
     assert "_2k" not in fa.describe_launch(3, 1, 8, 64, 1000, 128, False)             # split-KV's
     assert "_2k" not in fa.describe_launch(3, 1, 32, 2048, 2048, 128, False)          # whole rounds
     assert "_2k" not in fa.describe_launch(3, 1, 8, 1000, 1000, 128, True, dtype=fa.DTYPE_BF16)
+
+
+def test_folded_only_where_faster():
+    """Causal calls on which the folded grid was measured slower (us: the other
+    plan, folded), and calls that need no workspace."""
+    def plan(variant, *a):
+        return fa.describe_launch(variant, 1, *a, True)
+    assert "fa_merge" in plan(3, 48, 220, 2808, 200)     # key split 40.9, 49.5
+    assert "fa_merge" in plan(2, 41, 273, 273, 256)      # 53.8, 59.5
+    assert "stream_per" in plan(3, 26, 811, 933, 160)    # 119.5, 128.9
+    assert "stream_per" in plan(2, 20, 922, 922, 72)     # 64.5, 71.2
+    assert "stream_per" in plan(2, 2, 8350, 391, 128)    # 52.4, 61.3
+    for variant, bh, sq, sk, d in ((2, 3, 1901, 185, 200), (3, 2, 14032, 907, 256), (3, 3, 8071, 446, 256)):
+        assert "workspace" not in plan(variant, bh, sq, sk, d), (bh, sq, sk, d)
