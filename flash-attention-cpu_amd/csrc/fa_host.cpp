@@ -438,7 +438,8 @@ int make_plan(int variant, const void* q, const void* k, const void* v, const fl
             if (short2) n = 1;
             size_t len = ((sk + n - 1) / n + 63) / 64 * 64;
             n = (sk + len - 1) / len;
-            if (n <= (size_t)kMaxSplits && len <= imax && bh * n <= imax && bh * sq <= imax &&
+            // (the kernel's key indices, up to three blocks of 64 past the last split, are 32-bit)
+            if (n <= (size_t)kMaxSplits && n * len + 256 <= imax && bh * n <= imax && bh * sq <= imax &&
                 !(short2 && (sq > 16 || D == 256))) {
                 if (D == 128) {
                     plan->first.name += "s";

@@ -67,3 +67,15 @@ def test_few_rows_are_planned_only_for_their_calls():
                   plan(256, 16, 8192, 128, True), plan(256, 16, 255, 128, False),     # causal, few keys
                   plan(256, 16, 8192, 100, False), plan(256, 16, 4096, 32, False)):   # scalar loads, D = 32
         assert not other.split()[0].endswith("s"), other
+
+
+def test_few_rows_keep_their_key_indices_in_range():
+    """The streaming body's key indices, up to 256 past the last split's end, are
+    32-bit: key counts within that of 2^31 stay with the other kernels."""
+    def plan(sk, d):
+        return fa.describe_launch(2, 1, 1, 16, sk, d, False, dtype=fa.DTYPE_BF16)
+    for sk in (2**31 - 1, 2**31 - 255, 2**31 - 256):
+        assert "_rows" not in plan(sk, 40) and "splits=256 " not in plan(sk, 40), plan(sk, 40)
+    p = plan(2**31 - 2**15, 40)
+    assert p.startswith("fa_prefill_lp_bf16_d64_2_rows grid=256x1x1 "), p
+    assert "splits=256 split_len=8388480 " in p   # 2^31 - 2^15
