@@ -594,7 +594,13 @@ int make_plan(int variant, const void* q, const void* k, const void* v, const fl
                 const double fix = D == 32 ? 3.5 : D == 64 ? 3.6 : D == 128 ? 5.0 : 7.5;
                 const double plain = D == 32 ? 0.65 : D == 64 ? 0.80 : D == 128 ? (two ? 1.25 : 1.07) : 1.73;
                 const double split = D == 256 ? 1.9 : 1.19 * plain;
-                best = fix + plain * keys;
+                // Up to 64 queries K and V are most of an unsplit workgroup's work:
+                // the us that their bytes add (per MB; 90 x 17 x 3396 d256 99
+                // us in 64-row workgroups, 74 on the key split; 126 x 64 x 6730
+                // d128 109, 93; 118 x 52 x 10383 d64 98, 71)
+                const double bytes = causal || sq > 64 || D == 32 ? 0.0
+                                     : (D == 256 ? 0.03e-6 : 0.05e-6) * (double)bh * (double)d * (4.0 * (double)sk + 6.0 * (double)sq);
+                best = fix + plain * keys + bytes;
                 size_t wide = 0, wide_blocks = 0;   // rows and blocks (pairs of half blocks) per slice
                 bool wide_fold = false;
                 // (up to 128 keys a block has two stages; causal, up to three the
@@ -610,7 +616,7 @@ int make_plan(int variant, const void* q, const void* k, const void* v, const fl
                         const size_t half = f.rows / 2, nhb = (sq + half - 1) / half;
                         const bool fold = causal && nhb >= 2;
                         const size_t nb = (nhb + 1) / 2;
-                        const double t = f.fixed + (fold ? f.causal64 : f.key64) * keys;
+                        const double t = f.fixed + (fold ? f.causal64 : f.key64) * keys + bytes;
                         if (nb * bh <= (size_t)num_cus && t < best) {
                             best = t;
                             wide = f.rows;

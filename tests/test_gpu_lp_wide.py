@@ -108,3 +108,17 @@ def test_short_causal_calls_keep_the_plain_kernel():
                           (4, 6159, 255, 64)):      # 7.7, 8.5
         plan = fa.describe_launch(2, 1, bh, sq, sk, d, True, dtype=fa.DTYPE_BF16)
         assert "_t1 " in plan, (bh, sq, sk, d, plan)
+
+
+def test_few_queries_over_long_keys_are_split():
+    """Calls of up to 64 queries that are mostly K and V reads, measured slower
+    on unsplit 64-row workgroups (bf16, us: key split, workgroups)."""
+    for bh, sq, sk, d in ((90, 17, 3396, 256),      # 74, 99
+                          (102, 32, 3902, 256),     # 89, 122
+                          (126, 64, 6730, 128),     # 93, 109
+                          (118, 52, 10383, 64)):    # 71, 98
+        plan = fa.describe_launch(2, 1, bh, sq, sk, d, False, dtype=fa.DTYPE_BF16)
+        assert "; fa_merge" in plan, (bh, sq, sk, d, plan)
+    for bh, sq, sk, d in ((216, 33, 388, 64), (147, 17, 4291, 200)):   # workgroups 7.6 (9.1), 118 (121)
+        plan = fa.describe_launch(2, 1, bh, sq, sk, d, False, dtype=fa.DTYPE_BF16)
+        assert "_t1r64 " in plan, (bh, sq, sk, d, plan)
