@@ -438,9 +438,14 @@ int make_plan(int variant, const void* q, const void* k, const void* v, const fl
             if (short2) n = 1;
             size_t len = ((sk + n - 1) / n + 63) / 64 * 64;
             n = (sk + len - 1) / len;
+            // up to eight short splits on few CUs (D = 256, or two tiles at
+            // D = 128): the key split's 64-key stages are through sooner than
+            // the waves' 16-key blocks (7 x 8 x 2050 d256 18.2 us here, 16.2
+            // split; 6 x 32 x 1416 d128 15.0, 13.5)
+            const bool short8 = len < 384 && n <= 8 && (D == 256 ? n >= 4 && bh * n < 64 : D == 128 && sq > 16 && n >= 5 && bh * n < 40);
             // (the kernel's key indices, up to three blocks of 64 past the last split, are 32-bit)
             if (n <= (size_t)kMaxSplits && n * len + 256 <= imax && bh * n <= imax && bh * sq <= imax &&
-                !(short2 && (sq > 16 || D == 256))) {
+                !(short2 && (sq > 16 || D == 256)) && !short8) {
                 if (D == 128) {
                     plan->first.name += "s";
                 } else {

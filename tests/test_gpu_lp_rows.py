@@ -27,7 +27,7 @@ def inputs(name, n, seed):
 # bh, sq, sk, d: one and several splits; 16-row tiles of 1 .. 16 rows; keys that
 # end inside a 16-key block, a wave's last block and a split; d < D
 SHAPES = [
-    (2, 2, 256, 128), (3, 16, 1000, 128), (2, 17, 777, 128), (1, 32, 4096, 128), (300, 5, 259, 64),
+    (2, 2, 256, 128), (3, 16, 1000, 128), (2, 17, 3777, 128), (1, 32, 4096, 128), (300, 5, 259, 64),
     (40, 31, 2047, 64), (2, 7, 300, 40), (3, 9, 513, 96), (2, 16, 4000, 256), (3, 3, 271, 200), (130, 4, 2100, 128),
 ]
 
@@ -79,3 +79,17 @@ def test_few_rows_keep_their_key_indices_in_range():
     p = plan(2**31 - 2**15, 40)
     assert p.startswith("fa_prefill_lp_bf16_d64_2_rows grid=256x1x1 "), p
     assert "splits=256 split_len=8388480 " in p   # 2^31 - 2^15
+
+
+def test_few_short_splits_keep_the_key_split():
+    """Two to eight splits of under 384 keys on few CUs were measured slower on
+    the streaming body (bf16, us: key split, streaming body)."""
+    def plan(*a):
+        return fa.describe_launch(2, 1, *a, False, dtype=fa.DTYPE_BF16)
+    for bh, sq, sk, d in ((7, 8, 2050, 256), (1, 7, 1979, 256)):      # 16.2, 18.2; 15.2, 17.6
+        assert plan(bh, sq, sk, d).startswith("fa_prefill_lp_bf16_d256_2_t1s "), (bh, sq, sk, d)
+    for bh, sq, sk in ((1, 32, 1344), (6, 32, 1416)):                 # 13.3, 14.7; 13.5, 15.0
+        p = plan(bh, sq, sk, 128)
+        n = -(-sk // 256)   # the key split's own: 256 keys, not the streaming body's 320
+        assert p.startswith(f"fa_prefill_lp_bf16_d128_2_t2s grid={n * bh}x1x1 ") and "split_len=256 " in p, p
+    assert "_d256_2_rows " in plan(1, 2, 2756, 256) and "_d256_2_rows " in plan(42, 2, 1514, 256)
