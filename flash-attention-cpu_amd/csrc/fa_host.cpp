@@ -636,6 +636,11 @@ int make_plan(int variant, const void* q, const void* k, const void* v, const fl
                 // without a workspace (captured on any stream, overlapping others
                 // in the allocation-free form) does.
                 bool uneven = false;
+                // At D = 32 four workgroups fit a CU and the partials of whole
+                // blocks weigh more: us per 64 keys by workgroups per CU (1 x
+                // 19305^2 d24 121.3 in three splits, 104.6 in five; causal 2 x
+                // 12155^2 66.8 with two workgroups per CU, 61.3 with three)
+                static constexpr double round32[4] = {0.71, 1.03, 1.37, 1.85};
                 for (size_t R = 1; R <= 4 && nqb * bh < (size_t)num_cus; ++R) {
                     // the shortest split whose workgroups fit R per CU
                     const size_t slots = R * (size_t)num_cus;
@@ -658,7 +663,8 @@ int make_plan(int variant, const void* q, const void* k, const void* v, const fl
                     const double turns = D <= 128 ? (n <= cus ? 1.0 : pair * std::ceil(n / (2.0 * cus))) : std::ceil(n / cus);
                     double part = n * 128.0 * (4.0 * D + 8.0) * 2.0 / 4.0e6;
                     if (D == 256 && n <= cus) part = std::min(part, 9.0);
-                    const double t = turns * (fix + split * (double)lo) + 5.5 + part;
+                    double t = turns * (fix + split * (double)lo) + 5.5 + part;
+                    if (D == 32 && sq > 64) t = 8.4 + round32[R - 1] * (double)lo + 2.0 * part;
                     if (t < best) {
                         best = t;
                         per = lo;

@@ -122,3 +122,12 @@ def test_few_queries_over_long_keys_are_split():
     for bh, sq, sk, d in ((216, 33, 388, 64), (147, 17, 4291, 200)):   # workgroups 7.6 (9.1), 118 (121)
         plan = fa.describe_launch(2, 1, bh, sq, sk, d, False, dtype=fa.DTYPE_BF16)
         assert "_t1r64 " in plan, (bh, sq, sk, d, plan)
+
+
+def test_narrow_heads_fill_the_cus_with_splits():
+    """D = 32, whose workgroups fit four to a CU (bf16, us: two per CU, three)."""
+    def plan(*a):
+        return fa.describe_launch(2, 1, *a, dtype=fa.DTYPE_BF16)
+    assert "grid=755x1x1" in plan(1, 19305, 19305, 24, False)     # 121.3, 104.6
+    assert "grid=768x1x1" in plan(2, 12155, 12155, 32, True)      # 66.8, 61.3
+    assert "grid=252x1x1" in plan(6, 3, 31536, 32, False)         # few rows: one per CU 20.2, three 33.8
