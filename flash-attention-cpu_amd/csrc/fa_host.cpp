@@ -672,28 +672,33 @@ int make_plan(int variant, const void* q, const void* k, const void* v, const fl
                 }
                 if (!uneven) per = 0;
                 if (per > 0) wide = 0;
-                // Causal, few keys on a nearly full grid: what the estimates above
-                // leave out decides between the small workgroups (128 rows, 96
-                // at D = 128) and the plain kernel -- the bytes of the first
-                // fetches and last stores (per MB of Q, K, V and O) and, with
-                // fewer keys than queries, the keys that both half blocks of a
-                // pair see.  Fitted to 440 shapes (3 .. 7 % rms).  Plain against
-                // the workgroups that the estimates above take, us: 114 x 210^2
-                // d128 10.2 / 12.3, 93 x 226^2 10.2 / 11.9, 43 x 604 x 243 12.1 /
-                // 13.9, 91 x 204 x 1712 d64 6.9 / 8.0; the workgroups stay from
-                // about 700 keys on at D = 128 and 500 at 64.  (64 rows, and 96 at
-                // D = 64, stay: 0.93 .. 1.0 of plain from 208 keys on.)
-                if (causal && (wide == 128 || (wide == 96 && D == 128))) {
-                    const struct { double fixed, both64, long64, mb; } us[3] = {{4.9, 0.62, 0.425, 0.08}, {5.5, 0.78, 0.61, 0.10}, {6.0, 0.95, 0.63, 0.12}};
-                    const auto& f = us[D == 64 ? 0 : wide == 96 ? 1 : 2];
-                    const size_t half = wide / 2, nhb = (sq + half - 1) / half;
-                    const double end = (double)std::min(sk, nhb * half);                       // longest pair's
-                    const double mid = (double)std::min(sk, ((nhb - 1) / 2 + 1) * half);       // middle pair's short half
-                    const double mb = (double)bh * (double)d * 1e-6 *
-                                      (6.0 * (double)sq + 4.0 * (double)std::min(sk, nqb * rows));
-                    const double t = f.fixed + f.mb * mb + (f.long64 * end + std::max(0.0, f.both64 - f.long64) *
-                                                                                   std::max(0.0, 2.0 * mid - end)) / 64.0;
-                    if (t >= (D == 128 ? 3.5 + 1.09 * keys + 0.08 * mb : 3.2 + 0.80 * keys + 0.065 * mb)) wide = 0;
+                // Causal, few keys or a nearly full grid: what the estimates above
+                // leave out decides between the small workgroups and the plain
+                // kernel -- the bytes of the first fetches and last stores (per
+                // MB of Q, K, V and O), the keys that both half blocks of a pair
+                // see where there are fewer keys than queries, and the stages that
+                // the last query needs (64 keys plain, 128 in the workgroups).
+                // Fitted to 1450 pairs of times (choices within 0.3 % of the
+                // best in the geometric mean).  Plain against the workgroups that
+                // the estimates above take, us: 114 x 210^2 d128 10.2 / 12.3, 93 x
+                // 226^2 10.2 / 11.9, 43 x 604 x 243 12.1 / 13.9, 88 x 150 x 271
+                // 8.2 / 9.6, 91 x 204 x 1712 d64 6.9 / 8.0; the workgroups stay from
+                // about 700 keys on at D = 128 and 500 at 64.
+                if (wide && causal && D <= 128) {
+                    // plain: the fixed cost of the plain kernel beside it (d < 128 at
+                    // D = 128, whose left out columns save it less, pad more)
+                    const struct { double fixed, both64, long64, mb, plain, pad; } us[2][3] = {   // 64, 96, 128 rows
+                        {{4.5, 0.39, 0.405, 0.045, 3.9, 0.0}, {4.6, 0.52, 0.41, 0.06, 3.7, 0.0}, {4.9, 0.62, 0.425, 0.08, 3.3, 0.0}},
+                        {{5.5, 0.58, 0.54, 0.09, 3.7, 1.3}, {5.5, 0.78, 0.61, 0.10, 3.7, 1.3}, {6.0, 0.95, 0.63, 0.12, 3.7, 0.6}}};
+                    const auto& f = us[D == 128][wide / 32 - 2];
+                    const size_t half = wide / 2, nhb = (sq + half - 1) / half, end = std::min(sk, sq);
+                    const double mid = (double)std::min(end, ((nhb - 1) / 2 + 1) * half);   // middle pair's short half
+                    const double mb = (double)bh * (double)d * 1e-6 * (6.0 * (double)sq + 4.0 * (double)end);
+                    const double t = f.fixed + f.mb * mb + f.long64 * 2.0 * (double)((end + 127) / 128) +
+                                     std::max(0.0, f.both64 - f.long64) * std::max(0.0, 2.0 * mid - (double)end) / 64.0;
+                    const double stages = (double)((end + 63) / 64);
+                    const double pl = f.plain + (d < 128 ? f.pad : 0.0) + (D == 128 ? 1.09 * stages + 0.08 * mb : 0.80 * stages + 0.065 * mb);
+                    if (t >= pl) wide = 0;
                 }
                 if (wide) {
                     std::snprintf(buf, sizeof(buf), "fa_prefill_lp_%s_d%d_2_t1r%d", dtype == FA_DTYPE_BF16 ? "bf16" : "f16", D,

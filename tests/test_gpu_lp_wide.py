@@ -104,10 +104,15 @@ def test_short_causal_calls_keep_the_plain_kernel():
                           (93, 226, 226, 128),      # 10.2, 11.9
                           (43, 604, 243, 128),      # 12.1, 13.9
                           (53, 397, 397, 128),      # 13.5, 14.5
+                          (88, 150, 271, 128),      # 8.2, 9.6 (no query sees keys past 150)
+                          (1, 160, 8936, 128),      # 7.3, 8.0
                           (91, 204, 1712, 64),      # 6.9, 8.0
                           (4, 6159, 255, 64)):      # 7.7, 8.5
         plan = fa.describe_launch(2, 1, bh, sq, sk, d, True, dtype=fa.DTYPE_BF16)
         assert "_t1 " in plan, (bh, sq, sk, d, plan)
+    for bh, sq, sk, d in ((32, 139, 677, 72), (8, 175, 682, 72)):   # 7.8, 6.8; 7.7, 6.7
+        plan = fa.describe_launch(2, 1, bh, sq, sk, d, True, dtype=fa.DTYPE_BF16)
+        assert "_t1r64 " in plan, (bh, sq, sk, d, plan)
 
 
 def test_few_queries_over_long_keys_are_split():
