@@ -771,7 +771,11 @@ int make_plan(int variant, const void* q, const void* k, const void* v, const fl
                 const auto& o = u[stream ? 2 : 1];
                 const size_t tiles = stream ? (s_wgs + bh * nqb - 1) * (rows / 16) : bh * nqt * ((max_st + per - 1) / per);
                 const bool large = tiles * (16 * (size_t)D + 32) * sizeof(float) > FA_SCRATCH_BYTES;
-                fold_ok = keys <= best && (large || u[0].fixed + u[0].key * pair <= o.fixed + o.key * best);
+                // scalar loads slow the folded grid by more than the splits (1.05
+                // .. 1.2 times more: 5 x 6239^2 d62 v3 380 us folded, 310 on the
+                // stream split; 150 such calls 0.913 on their splits)
+                const double slower = vec || D == 32 ? 1.0 : variant == 3 ? 1.2 : D == 64 ? 1.05 : 1.15;
+                fold_ok = keys <= best && (large || slower * (u[0].fixed + u[0].key * pair) <= o.fixed + o.key * best);
                 if (fold_ok) {
                     best = keys;
                     per = 0;

@@ -117,5 +117,7 @@ def test_folded_only_where_faster():
     assert "stream_per" in plan(3, 26, 811, 933, 160)    # 119.5, 128.9
     assert "stream_per" in plan(2, 20, 922, 922, 72)     # 64.5, 71.2
     assert "stream_per" in plan(2, 2, 8350, 391, 128)    # 52.4, 61.3
+    assert "stream_per" in plan(3, 5, 6239, 6239, 62)    # scalar loads: 310, 380
+    assert "fa_merge" in plan(3, 26, 534, 534, 62)       # 34.4, 39.9
     for variant, bh, sq, sk, d in ((2, 3, 1901, 185, 200), (3, 2, 14032, 907, 256), (3, 3, 8071, 446, 256)):
         assert "workspace" not in plan(variant, bh, sq, sk, d), (bh, sq, sk, d)
