@@ -496,7 +496,11 @@ int make_plan(int variant, const void* q, const void* k, const void* v, const fl
         // (map_block), and folding would make its last round a full one.
         // Measured on MI355X (v3, causal): 16 x 2048^2 d128 247 -> 148 us,
         // 32 x 1024^2 d128 126 -> 81, 16 x 2048^2 d64 130 -> 79.
-        bool fold_ok = !lp && causal_skip && D <= kMaxDNarrow && nqb >= 2 && nqb * bh <= (size_t)num_cus;
+        // (v2 with 128-bit operands, whose folded grids run v3's kernel, from 128
+        // keys on: two stages start sooner in its own, 24 x 937 x 47 d100 13.5
+        // against 15.2 us, 56 x 162 x 27 d72 12.0 against 13.4)
+        bool fold_ok = !lp && causal_skip && D <= kMaxDNarrow && nqb >= 2 && nqb * bh <= (size_t)num_cus &&
+                       !(variant == 2 && vec && sk <= 128 && (D == 64 || D == 128));
         // f32 v3 with 128-bit DMA and d = D = 128: pair query blocks nqb-1-r
         // and r in one workgroup (equal causal work per workgroup; the
         // second block's loads overlap the first's last step) when the

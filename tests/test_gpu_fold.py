@@ -30,7 +30,7 @@ FOLD = [
     (85, 320, 320, 64),      # 5 full ones
     (128, 129, 129, 32),     # 3, one row in the last
     (64, 449, 449, 256),     # 8, one row in the last
-    (85, 300, 100, 128),     # keys end inside the second half block
+    (85, 300, 140, 128),     # keys end inside the third half block
     (85, 300, 700, 64),      # keys past the last query
     (85, 300, 300, 90),      # scalar loads (d % 4 != 0)
 ]
@@ -119,5 +119,8 @@ def test_folded_only_where_faster():
     assert "stream_per" in plan(2, 2, 8350, 391, 128)    # 52.4, 61.3
     assert "stream_per" in plan(3, 5, 6239, 6239, 62)    # scalar loads: 310, 380
     assert "fa_merge" in plan(3, 26, 534, 534, 62)       # 34.4, 39.9
+    # v2, up to 128 keys: its own kernel 13.5, 12.0; folded (v3's) 15.2, 13.4
+    assert plan(2, 24, 937, 47, 100).startswith("fa_prefill_v2_d128_1 ")
+    assert plan(2, 56, 162, 27, 72).startswith("fa_prefill_v2_d128_1 ")
     for variant, bh, sq, sk, d in ((2, 3, 1901, 185, 200), (3, 2, 14032, 907, 256), (3, 3, 8071, 446, 256)):
         assert "workspace" not in plan(variant, bh, sq, sk, d), (bh, sq, sk, d)
