@@ -645,6 +645,11 @@ int make_plan(int variant, const void* q, const void* k, const void* v, const fl
                 // 19305^2 d24 121.3 in three splits, 104.6 in five; causal 2 x
                 // 12155^2 66.8 with two workgroups per CU, 61.3 with three)
                 static constexpr double round32[4] = {0.71, 1.03, 1.37, 1.85};
+                // up to 64 queries K and V are read from memory and the merge
+                // walks the splits: fixed + per 64 keys + per MB (177 x 39 x 5259
+                // 51.5 us in two splits, 40.0 in four)
+                static constexpr struct { double fixed, key64, mb; } rows32[4] = {
+                    {9.0, 0.6, 0.06}, {10.0, 0.6, 0.14}, {11.0, 0.3, 0.23}, {11.5, 0.2, 0.26}};
                 for (size_t R = 1; R <= 4 && nqb * bh < (size_t)num_cus; ++R) {
                     // the shortest split whose workgroups fit R per CU
                     const size_t slots = R * (size_t)num_cus;
@@ -668,7 +673,12 @@ int make_plan(int variant, const void* q, const void* k, const void* v, const fl
                     double part = n * 128.0 * (4.0 * D + 8.0) * 2.0 / 4.0e6;
                     if (D == 256 && n <= cus) part = std::min(part, 9.0);
                     double t = turns * (fix + split * (double)lo) + 5.5 + part;
-                    if (D == 32 && sq > 64) t = 8.4 + round32[R - 1] * (double)lo + 2.0 * part;
+                    if (D == 32 && sq > 64) {
+                        t = 8.4 + round32[R - 1] * (double)lo + 2.0 * part;
+                    } else if (D == 32 && !causal) {
+                        t = rows32[R - 1].fixed + rows32[R - 1].key64 * (double)lo + 0.115 * (double)((max_st + lo - 1) / lo) +
+                            rows32[R - 1].mb * 1e-6 * (double)bh * (double)d * (4.0 * (double)sk + 6.0 * (double)sq);
+                    }
                     if (t < best) {
                         best = t;
                         per = lo;

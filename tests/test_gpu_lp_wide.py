@@ -136,3 +136,4 @@ def test_narrow_heads_fill_the_cus_with_splits():
     assert "grid=755x1x1" in plan(1, 19305, 19305, 24, False)     # 121.3, 104.6
     assert "grid=768x1x1" in plan(2, 12155, 12155, 32, True)      # 66.8, 61.3
     assert "grid=252x1x1" in plan(6, 3, 31536, 32, False)         # few rows: one per CU 20.2, three 33.8
+    assert "grid=708x1x1" in plan(177, 39, 5259, 32, False)       # two 51.5, four 40.0
