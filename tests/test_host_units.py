@@ -6,6 +6,10 @@ leaves a gap sends stale bytes of the pinned ring to the device, so every
 byte count -- in particular the odd 16-bit ones, 2 * (128m + 1) -- must be
 covered exactly once.  The header is compiled here with g++ on its own.
 
+The launch planner's fold and few_rows flags, which pick a body or a row order
+inside a kernel and so do not show in its name or grid, are read from
+csrc/fa_host.cpp itself for the shapes of the GPU tests that mean to run them.
+
 Also the arithmetic behind one 16-bit GPU test input (f16 probabilities in
 the subnormal range).
 """
@@ -16,6 +20,9 @@ import subprocess
 
 import numpy as np
 
+import test_gpu_fold
+import test_gpu_lp_rows
+import test_gpu_lp_wide
 from fa_testutil import long_row_f16_case
 
 ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
@@ -72,6 +79,49 @@ def test_copy_pool_partition_covers_every_byte(tmp_path):
                    check=True)
     r = subprocess.run([str(exe)], capture_output=True, text=True)
     assert r.returncode == 0 and r.stdout.strip().endswith("OK"), r.stdout
+
+
+PLAN = r"""
+#include "fa_host.cpp"
+int fa_scratch_init(int) { return FA_ERR_SCRATCH; }
+void* fa_scratch_ptr(int) { return nullptr; }
+
+// stdin: variant dtype bh sq sk d causal; stdout: fold few_rows kernel
+int main() {
+    int variant, dtype, causal;
+    size_t bh, sq, sk, d;
+    static const float dummy[4] __attribute__((aligned(16))) = {0, 0, 0, 0};
+    while (std::scanf("%d %d %zu %zu %zu %zu %d", &variant, &dtype, &bh, &sq, &sk, &d, &causal) == 7) {
+        fa_launch_opts opts = {0.0f, FA_PATH_AUTO, 0, dtype};
+        Plan plan;
+        if (make_plan(variant, dummy, dummy, dummy, dummy, bh, sq, sk, d, causal, &opts, 256, &plan) != FA_OK) return 1;
+        std::printf("%d %d %s\n", plan.p.fold, plan.p.few_rows, plan.first.name.c_str());
+    }
+    return 0;
+}
+"""
+
+
+def test_plans_fold_and_stream_rows_where_the_gpu_tests_say(tmp_path):
+    rocm = os.environ.get("ROCM_PATH", "/opt/rocm")
+    src, exe = tmp_path / "plan.cpp", tmp_path / "plan"
+    src.write_text(PLAN)
+    subprocess.run([os.path.join(rocm, "llvm", "bin", "clang++"), "-std=c++17", "-O1", "-w", "-D__HIP_PLATFORM_AMD__",
+                    "-I", os.path.join(rocm, "include"), "-I", CSRC, str(src), "-L", os.path.join(rocm, "lib"),
+                    "-lamdhip64", "-Wl,-rpath," + os.path.join(rocm, "lib"), "-lpthread", "-ldl", "-o", str(exe)],
+                   check=True)
+    calls = [((v, 0, *s, 1), (1, 0)) for s in test_gpu_fold.FOLD for v in (2, 3)]
+    calls += [((2, dt, *s, 0), (0, 1)) for s in test_gpu_lp_rows.SHAPES for dt in (1, 2)]
+    calls += [((2, dt, *s[1:5], int(s[5])), (int(s[5]), 0)) for s in test_gpu_lp_wide.SHAPES for dt in (1, 2)]
+    # neither: the key split by the streaming body's kernel name, more rows, few keys, unfolded small blocks
+    calls += [((2, 1, 6, 32, 1416, 128, 0), (0, 0)), ((2, 1, 8, 48, 4096, 128, 0), (0, 0)),
+              ((2, 1, 8, 16, 255, 128, 0), (0, 0)), ((3, 0, 32, 2048, 2048, 120, 1), (0, 0)),
+              ((1, 0, 128, 256, 256, 64, 1), (0, 0)), ((2, 1, 114, 210, 210, 128, 1), (0, 0))]
+    text = "".join(" ".join(str(x) for x in c) + "\n" for c, _ in calls)
+    out = subprocess.run([str(exe)], input=text, capture_output=True, text=True, check=True).stdout.splitlines()
+    assert len(out) == len(calls)
+    for (call, flags), line in zip(calls, out):
+        assert tuple(int(x) for x in line.split()[:2]) == flags, (call, line)
 
 
 def test_long_row_f16_case_breaks_the_bound_without_scaling():
