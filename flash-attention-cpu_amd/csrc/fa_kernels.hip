@@ -500,7 +500,9 @@ __device__ __forceinline__ void prefill_segment(const FaParams& p, const Prefill
     // DMA: the stage image is SK rows of LD/4 chunks (the last ones are the
     // pad); run R = i*FW + f (64 chunks = 1 KB) is written by filling wave f,
     // lane L fetching the global chunk that belongs at image position 64R + L
-    // (columns past d and pad slots fetch column 0).  Every stage is fetched
+    // (pad slots, never read, fetch column 0; columns past d lie out of the
+    // buffer's range and read as zeros: a copied infinite element there would
+    // meet Q's zero columns and make the score NaN).  Every stage is fetched
     // with buffer loads: a per-stage buffer resource (base = the stage's
     // first row, range ending at seq_k, in SGPRs) and per-lane byte offsets
     // that are the same for every stage, computed once below -- no per-stage
@@ -524,7 +526,7 @@ __device__ __forceinline__ void prefill_segment(const FaParams& p, const Prefill
         for (int i = 0; i < NI; ++i) {
             const int pos = (i * FW + fwave) * 64 + lane;
             const int r = pos / RCH, cidx = pos % RCH;
-            const int col = (cidx < CPR && 4 * cidx < d) ? 4 * cidx : 0;
+            const int col = (cidx < CPR && 4 * cidx < d) ? 4 * cidx : (cidx < CPR ? 1 << 28 : 0);
             voff[i] = (fwave >= 0 && pos < TOTAL) ? 4 * (r * d + col) : -1;   // -1: lane past the image
         }
     };
@@ -1667,15 +1669,15 @@ __device__ __forceinline__ void decode_body(const FaParams& p) {
         // branches around loads), so the wave's vmcnt counts are exact and
         // the waits below name exactly the block they need.
         // Per-lane DMA offsets, the same for every block: image position
-        // 64 i + lane is chunk pos % KCH of row pos / KCH (pad chunks and
-        // columns past d fetch column 0); lanes past the image fetch out of
-        // range (zeros) into the slot's slack after the image.
+        // 64 i + lane is chunk pos % KCH of row pos / KCH (pad chunks fetch
+        // column 0); columns past d and lanes past the image (into the slot's
+        // slack) fetch out of range (zeros).
         int kvoff[KRUNS];
 #pragma unroll
         for (int i = 0; i < KRUNS; ++i) {
             const int pos = 64 * i + lane;
             const int r = pos / KCH, ci = pos % KCH;
-            const int col = (ci < D / 4 && 4 * ci < d) ? 4 * ci : 0;
+            const int col = (ci < D / 4 && 4 * ci < d) ? 4 * ci : (ci < D / 4 ? 1 << 28 : 0);
             kvoff[i] = pos < KTOT ? 4 * (r * d + col) : 0x40000000;
         }
         // V (A operand of O^T): rows 4lg + r, columns 64hh + 4lr; columns
