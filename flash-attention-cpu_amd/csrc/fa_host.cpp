@@ -425,7 +425,12 @@ int make_plan(int variant, const void* q, const void* k, const void* v, const fl
         // 5.1 against 5.9 us.)  Measured on MI355X against the key-split
         // prefill, bf16, us: 32 x 16 x 32768 d128 101.8 -> 83.2, 256 x 16 x
         // 8192 186 -> 153 (7.0 TB/s), d64 114 -> 77, d256 32 x 16 x 32768 184
-        // -> 160; two workgroups per CU 83.8 / 161 / 84 / 187.  Two short
+        // -> 160; two workgroups per CU 83.8 / 161 / 84 / 187.  Slice counts
+        // that leave CUs idle gain as well: 65 x 16 x 8192 d128 56.0 -> 46.0,
+        // 129 109.6 -> 92.2, 255 194.9 -> 154.2, 129 x 4 x 16384 d64 115.7 ->
+        // 115.6, 129 x 16 x 4096 d256 120.7 -> 94.0.  At D = 256 a second
+        // tile of rows (17 .. 32) loses below about 1400 keys a workgroup
+        // (8 x 24 x 24314 45.3 against the others' 40.0).  Two short
         // splits lose to one: 128 x 16 x 1024 16.7 against 14.9; with two
         // tiles or at D = 256 that one loses to the small grids' workgroups
         // below (64 x 32 x 674 15.7 against 11.5, 128 x 2 x 1630 d256 42.2
@@ -582,20 +587,20 @@ int make_plan(int variant, const void* q, const void* k, const void* v, const fl
                 per = (max_st + opts->num_splits - 1) / opts->num_splits;
             } else if (path == FA_PATH_AUTO && lp && vec && nqb * bh <= (size_t)num_cus) {
                 // 16-bit grids of at most one block per CU, estimated in us
-                // (MI355X, bf16; every shape of 1 .. 32 heads x 512 .. 4096
-                // within 15 %), fixed + per 64 keys: the plain kernel; 64, 96 or
+                // (MI355X, bf16), fixed + per 64 keys: the plain kernel; 64, 96 or
                 // 128 rows with 4, 2, 2 waves on each tile's keys (D = 64, 128;
                 // at D = 256, whose registers allow 8 waves, 64 with 2;
                 // causal: folded), where they all run at once; the key split,
                 // whose kernel is slower a stage (its segment loop) and which
                 // adds a merge launch and its partials, written and read back
                 // at 4 TB/s (at D = 256 and one workgroup per CU 9 us at most:
-                // 80 .. 256 workgroups, 11 .. 14 us with the merge launch).  us before -> now: 16 x 1500^2 d64 36.9 -> 17.7 (96
-                // rows; key split before), 16 x 1024^2 23.8 -> 11.3 and d128 36.5
-                // -> 16.4 (64), causal 8 x 2048^2 33.4 -> 24.1 (64), 16 x 2048^2
-                // 41.2 -> 30.1 and 8 x 4096^2 75.4 -> 50.0 (128; plain before);
-                // d256 16 x 1024^2 38.0 -> 27.6 (plain before), 8 x 2048^2 53.4
-                // -> 45.8 (key split before).
+                // 80 .. 256 workgroups, 11 .. 14 us with the merge launch).
+                // The small workgroups against the plan without them, us: 16 x
+                // 1500^2 d64 17.7 (96 rows) and 36.9 (key split), 16 x 1024^2
+                // 11.3 and 23.8, d128 16.4 (64) and 36.5; against plain, causal
+                // 8 x 2048^2 24.1 (64) and 33.4, 16 x 2048^2 30.1 and 41.2, 8 x
+                // 4096^2 50.0 (128) and 75.4, d256 16 x 1024^2 27.6 and 38.0;
+                // against the key split, d256 8 x 2048^2 45.8 and 53.4.
                 // The key split stays for few blocks of many keys: 1 x 2048^2
                 // d64 13.9 against 17.2.
                 const double cus = (double)num_cus, keys = (double)max_st;

@@ -20,7 +20,8 @@ typedef struct FaParams {
     int d;               // true d_head (kernels pad to D)
     int causal;          // top-left aligned: key j visible to query i iff j <= i
     float scale_log2e;   // (1/sqrt(d) computed in f32) * log2(e)
-    int nqb;             // prefill: query blocks of 128 rows
+    int nqb;             // prefill: query blocks of the launched kernel's rows per slice (folded:
+                         // workgroups, each of two half blocks)
     int nqt;             // split-KV: query tiles of 16 rows
     int num_splits;      // split-KV / key split: key splits per (bh, query tile)
     int split_len;       // keys per split (split-KV: multiple of 64; key split: of the stage)
@@ -32,11 +33,13 @@ typedef struct FaParams {
                          // block); 0 = plain longest-first order
     int two_blocks;      // f32 v3 prefill, d_head 128: each workgroup runs query blocks
                          // nqb-1-r and r of one (batch, head); nqb even, grid = bh * nqb / 2
-    int fold;            // f32 v2 / v3 prefill, causal: a workgroup's lower 64 rows are half block
-                         // nhb-1-r of the slice, its upper 64 rows half block r (equal work per
-                         // workgroup); 0 = 128 consecutive rows
-    int few_rows;        // 16-bit D = 128 split kernel: at most 32 query rows, num_splits workgroups per slice
-                         // stream split_len keys each
+    int fold;            // causal prefill, f32 v2 / v3 and the 16-bit kernels whose waves share a
+                         // tile's keys: a workgroup's lower half of rows is half block nhb-1-r of
+                         // the slice, its upper half is half block r (equal work per workgroup;
+                         // 16 .. 64 rows each); 0 = consecutive rows
+    int few_rows;        // 16-bit, at most 32 query rows: num_splits workgroups per slice stream
+                         // split_len keys each (set for every d_head; the D = 128 split kernel
+                         // branches on it, the _rows kernels do nothing else)
     int full_keys;       // v1: every query block visits all seq_k keys, causal or not (no
                          // causal skip), so the key split, the stream split and fa_merge
                          // count each block's keys as the whole key range

@@ -174,10 +174,14 @@ int fa_release_stream_workspace(void* stream);
  * normalisation and visit every key (no causal skip).  AUTO runs
  * decode steps -- seq_len_q <= 32, any batch and key count -- on split-KV
  * (the row-streaming kernel where it applies, else 16-row tiles; 16-bit
- * inputs on the row kernel for one query, on a streaming prefill kernel for
- * more), and prefills smaller than the GPU on smaller workgroups whose waves
- * share the keys of a query tile, on the stream split or on the key split,
- * whichever it estimates to be fastest.
+ * inputs on the row kernel for one query; for 2 .. 32 queries -- 16 where
+ * d_head > 128 -- on a streaming prefill kernel if non-causal, with 256 keys
+ * or more, d_head > 32, d_head % 8 == 0 and 16-byte aligned operands, unless
+ * that would run as a few short splits, which go to the small prefill grids
+ * below), and prefills smaller than the GPU on smaller workgroups whose
+ * waves share the keys of a query tile, on the stream split or on the key
+ * split, whichever it estimates to be fastest; a 16-bit grid that nearly
+ * fills the GPU runs without a workspace.
  * num_splits = 0 lets the library choose (at most 1024). */
 #define FA_PATH_AUTO 0
 #define FA_PATH_PREFILL 1
@@ -289,11 +293,10 @@ int fa_describe_launch(int variant, size_t batch, size_t heads, size_t seq_len_q
  *     back-to-back MFMAs of that kind and writes one checksum float to buf
  *     (bytes >= 128 x #CUs); *work = FLOP.
  *   FA_PROBE_COPY: copies the first bytes/2 of buf (whole 16-byte elements)
- *     onto the second half;
+ *     onto the second half; *work = bytes read + bytes written;
  *   FA_PROBE_READ: reads the first bytes/2 of buf (whole 16-byte elements),
  *     each workgroup one contiguous chunk, and writes nothing; *work = bytes
- *     read;
- *     *work = bytes read + bytes written. */
+ *     read. */
 #define FA_PROBE_MFMA_F32_32X32X2 0
 #define FA_PROBE_MFMA_F32_16X16X4 1
 #define FA_PROBE_MFMA_BF16_16X16X32 2
