@@ -1,6 +1,6 @@
 """Build the MI355X library in-tree.
 
-Outputs, next to this file (git-ignored, shipped to the GPU box with the tree):
+Outputs, next to this file (git-ignored, used in place):
   fa_kernels.hsaco  gfx950 code object with every kernel (hipcc --genco)
   libfa_hip.so      C ABI of include/fa_hip.h over the HIP runtime
 

@@ -46,14 +46,15 @@ constexpr int kRowsMaxQ = 4;        // row-streaming decode: most query rows
 
 // Host-slice staging: pageable host memory moves through a ring of pinned
 // buffers.  Host threads copy pageable <-> pinned while the DMA engine moves
-// the previous buffer.  Measured on the MI355X box: pageable hipMemcpyAsync
+// the previous buffer.  Measured (MI355X): pageable hipMemcpyAsync
 // 25 GB/s host-to-device and 16 GB/s device-to-host; staged through 16 MiB
 // pinned chunks with 4 host threads 54 GB/s both ways.
 constexpr size_t kStageChunk = size_t(16) << 20;
 constexpr int kStageBufs = 4;
 constexpr int kCopyThreads = 4;     // host threads per staging copy, the caller included
 constexpr size_t kCopySplitMin = size_t(1) << 20;   // smaller copies stay on the caller
-// Transfers below this many bytes take plain pageable copies: the ring's
+// Uploads (Q, K and V together) and outputs below this many bytes take plain
+// pageable copies: the ring's
 // per-chunk events cost more than they save on small calls (measured: a
 // 256 x 64 single-head call 78 -> 111 us through the ring).
 constexpr size_t kStageMinBytes = size_t(2) << 20;

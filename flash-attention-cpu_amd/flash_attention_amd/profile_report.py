@@ -26,19 +26,19 @@ import sys
 _PKG_DIR = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
 ROOT = os.path.dirname(_PKG_DIR)
 
-PMC_COMMANDS = """rocprofv3 --pmc SQ_VALU_MFMA_BUSY_CYCLES SQ_BUSY_CYCLES SQ_INSTS_VALU SQ_INSTS_MFMA SQ_WAVE_CYCLES SQ_WAIT_INST_ANY GRBM_GUI_ACTIVE -d gpurun_out/pmcA -o run -f csv -- python3 bench.py --steps 3 --warmup 1 --no-cpu-baseline
-rocprofv3 --pmc SQ_LDS_BANK_CONFLICT SQ_LDS_IDX_ACTIVE SQ_INSTS_LDS SQ_WAIT_INST_LDS SQ_LDS_ADDR_CONFLICT GRBM_GUI_ACTIVE -d gpurun_out/pmcB -o run -f csv -- python3 bench.py --steps 3 --warmup 1 --no-cpu-baseline
-cd flash-attention-cpu_amd && python3 -m flash_attention_amd.traffic --pmc-a ../gpurun_out/pmcA --pmc-b ../gpurun_out/pmcB --out ../profiles/pmc.json"""
+PMC_COMMANDS = """rocprofv3 --pmc SQ_VALU_MFMA_BUSY_CYCLES SQ_BUSY_CYCLES SQ_INSTS_VALU SQ_INSTS_MFMA SQ_WAVE_CYCLES SQ_WAIT_INST_ANY GRBM_GUI_ACTIVE -d out/pmcA -o run -f csv -- python3 bench.py --steps 3 --warmup 1 --no-cpu-baseline
+rocprofv3 --pmc SQ_LDS_BANK_CONFLICT SQ_LDS_IDX_ACTIVE SQ_INSTS_LDS SQ_WAIT_INST_LDS SQ_LDS_ADDR_CONFLICT GRBM_GUI_ACTIVE -d out/pmcB -o run -f csv -- python3 bench.py --steps 3 --warmup 1 --no-cpu-baseline
+cd flash-attention-cpu_amd && python3 -m flash_attention_amd.traffic --pmc-a ../out/pmcA --pmc-b ../out/pmcB --out ../profiles/pmc.json"""
 
-TRAFFIC_COMMANDS = """rocprofv3 --pmc FETCH_SIZE -d gpurun_out/tr_fetch -o run -f csv -- python3 bench.py --no-cpu-baseline --steps 5 --warmup 1
-rocprofv3 --pmc WRITE_SIZE -d gpurun_out/tr_write -o run -f csv -- python3 bench.py --no-cpu-baseline --steps 5 --warmup 1
-rocprofv3 --pmc FETCH_SIZE -d gpurun_out/tr_cf -o run -f csv -- python3 bench.py --calibrate-copy-mib 1024
-rocprofv3 --pmc WRITE_SIZE -d gpurun_out/tr_cw -o run -f csv -- python3 bench.py --calibrate-copy-mib 1024
-cd flash-attention-cpu_amd && python3 -m flash_attention_amd.traffic --fetch ../gpurun_out/tr_fetch \\
-    --write ../gpurun_out/tr_write --copy-fetch ../gpurun_out/tr_cf --copy-write ../gpurun_out/tr_cw \\
+TRAFFIC_COMMANDS = """rocprofv3 --pmc FETCH_SIZE -d out/tr_fetch -o run -f csv -- python3 bench.py --no-cpu-baseline --steps 5 --warmup 1
+rocprofv3 --pmc WRITE_SIZE -d out/tr_write -o run -f csv -- python3 bench.py --no-cpu-baseline --steps 5 --warmup 1
+rocprofv3 --pmc FETCH_SIZE -d out/tr_cf -o run -f csv -- python3 bench.py --calibrate-copy-mib 1024
+rocprofv3 --pmc WRITE_SIZE -d out/tr_cw -o run -f csv -- python3 bench.py --calibrate-copy-mib 1024
+cd flash-attention-cpu_amd && python3 -m flash_attention_amd.traffic --fetch ../out/tr_fetch \\
+    --write ../out/tr_write --copy-fetch ../out/tr_cf --copy-write ../out/tr_cw \\
     --copy-mib 1024 --out ../profiles/traffic.json"""
 
-TRACE_COMMANDS = """rocprofv3 --kernel-trace --stats -d gpurun_out/ks -o run -f csv -- python3 bench.py --no-cpu-baseline"""
+TRACE_COMMANDS = """rocprofv3 --kernel-trace --stats -d out/ks -o run -f csv -- python3 bench.py --no-cpu-baseline"""
 
 REPORT_COMMAND = ("cd flash-attention-cpu_amd && python3 -m flash_attention_amd.profile_report "
                   "--traffic ../profiles/traffic.json --pmc ../profiles/pmc.json --out-dir ../profiles")
@@ -185,7 +185,7 @@ def trace_markdown(run_dir: str, calls, src: str) -> str:
         f"Kernel sources sha256 `{src}`.  Commands (one MI355X, repo root):", "", "```",
         TRACE_COMMANDS,
         "cd flash-attention-cpu_amd && python3 -m flash_attention_amd.profile_report --traffic ../profiles/traffic.json "
-        "--pmc ../profiles/pmc.json --out-dir ../profiles --trace ../gpurun_out/ks",
+        "--pmc ../profiles/pmc.json --out-dir ../profiles --trace ../out/ks",
         "```", "",
         "The name-keyed `run_kernel_stats.csv` mixes launch sizes (one kernel serves several configs), so this",
         "table is the kernel trace grouped by kernel and launch size; library kernels only.  Call counts include",

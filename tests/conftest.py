@@ -15,4 +15,4 @@ for sub in ("", "flash-attention-cpu_amd", "oracle", "tests"):
 
 
 def pytest_configure(config):
-    config.addinivalue_line("markers", "gpu: needs an AMD MI355X (gfx950); runs on the GPU box")
+    config.addinivalue_line("markers", "gpu: needs an AMD MI355X (gfx950)")

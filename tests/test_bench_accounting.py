@@ -115,7 +115,7 @@ def _fake_configs():
 
 
 def test_summary_survives_a_2000_character_tail():
-    """The driver keeps the last few KB of stderr: the closing summary (one
+    """A reader may keep only the last few KB of stderr: the closing summary (one
     line per config, every variant with time, rate, % of peak and parity)
     must fit in 2000 characters."""
     lines = bench.summary_lines(_fake_configs())
@@ -131,7 +131,7 @@ def test_summary_survives_a_2000_character_tail():
 
 def test_json_line_stays_compact():
     """The one stdout JSON line (every config's figures in extra.configs) stays
-    well inside the driver's 16 KB stdout tail."""
+    well inside a 16 KB tail of stdout."""
     import json as _json
     line = _json.dumps({"metric": bench.METRIC, "extra": {"configs": _fake_configs()}}, separators=(",", ":"))
     assert len(line) < 9000, len(line)

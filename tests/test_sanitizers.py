@@ -1,6 +1,6 @@
 """AddressSanitizer + UndefinedBehaviorSanitizer builds of the CPU code.
 
-GPU code cannot be sanitised on this pool, so the checks cover what runs on
+GPU code is not sanitised, so the checks cover what runs on
 the host:
 
 * the host library's CPU-side paths -- flash-attention-cpu_amd/csrc/fa_host.cpp
